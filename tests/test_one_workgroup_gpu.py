@@ -1,0 +1,71 @@
+"""Solves inside one workgroup with the vertex state in LDS: sizes at the edges of what fits, of the
+hub handling and of the hand-over to the grid-wide kernels, against Dinic, certified."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def arcs_graph(mf, n, parts, s, t, seed, top=1000):
+    u = np.concatenate([np.broadcast_to(a, np.broadcast(a, b).shape).ravel() for a, b in parts])
+    v = np.concatenate([np.broadcast_to(b, np.broadcast(a, b).shape).ravel() for a, b in parts])
+    cap = np.random.default_rng(seed).integers(1, top + 1, size=u.size)
+    return mf.Graph.from_arcs(n, u, v, cap, s, t)
+
+
+def chains(mf, width, length, seed):
+    """width chains of length vertices into t; s feeds every vertex, so the first worklist holds
+    all of them while no BFS frontier is wider than width."""
+    n = width * length + 2
+    x = 2 + np.arange(width * length).reshape(length, width)
+    parts = [(np.array([0]), x.ravel()), (x[:-1], x[1:]), (x[-1], np.array([1]))]
+    parts.append((x[1:], np.roll(x[:-1], 1, axis=1)))  # and back, to the chain beside it
+    return arcs_graph(mf, n, parts, 0, 1, seed)
+
+
+def dense_layers(mf, k, layers, seed):
+    """Complete bipartite arcs between layers of k vertices: every inner vertex has 2k slots."""
+    x = 2 + np.arange(k * layers).reshape(layers, k)
+    parts = [(np.array([0]), x[0]), (x[-1], np.array([1]))]
+    parts += [(x[i][:, None], x[i + 1][None, :]) for i in range(layers - 1)]
+    return arcs_graph(mf, k * layers + 2, parts, 0, 1, seed)
+
+
+def check(mf, orc, ctx, g):
+    value = orc.dinic_maxflow(g)
+    tails = g.tails()
+    for layout in (mf.LAYOUT_BCSR, mf.LAYOUT_BCSR2, mf.LAYOUT_RCSR):
+        dg = ctx.upload(g, layout)
+        try:
+            for algo in (mf.ALGO_VC, mf.ALGO_TC):  # the second restores the residuals first
+                r = dg.solve(algo)
+                assert r.value == value and r.pushes > 0
+                assert orc.certify(g, dg.read_flow(return_excess=False), value,
+                                   preflow=True)[0] == "ok"
+                assert orc.certify(g, dg.read_flow(), value) == ("ok", value)
+                side = dg.read_cut()
+                assert g.cap[(side[tails] == 0) & (side[g.dst] == 1)].sum(dtype=np.int64) == value
+        finally:
+            dg.close()
+
+
+@pytest.mark.parametrize("width,length", [
+    (63, 17), (64, 16), (1, 300),  # bitmap words, single-vertex frontiers
+    (1500, 15),    # excesses in LDS, worklists longer than their lists
+    (1300, 19),    # about as many vertices as fit with their excesses
+    (1301, 20),    # more: excesses in global memory
+    (1500, 41),    # nearly as many as fit at all
+    (1600, 42),    # too many
+    (2048, 9), (2049, 9),  # the widest frontier that stays, and one more vertex
+])
+def test_chains(mf, orc, ctx, width, length):
+    check(mf, orc, ctx, chains(mf, width, length, seed=width + length))
+
+
+@pytest.mark.parametrize("k,layers", [
+    (47, 6), (48, 6), (49, 6),  # 94, 96 and 98 slots: the last are hubs
+    (130, 4),                   # hubs of one and a half rounds of a wave
+    (290, 3),                   # more hubs at a time than wait in LDS
+])
+def test_hubs(mf, orc, ctx, k, layers):
+    check(mf, orc, ctx, dense_layers(mf, k, layers, seed=k))

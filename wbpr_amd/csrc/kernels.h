@@ -65,6 +65,23 @@ struct LayoutBCSR {
       dirty[rk >> 3] = 1;
     }
   }
+  // A slot's push where nothing else touches its pair of residuals meanwhile: pair() loads what
+  // the push needs besides the slot's residual res, push_pair() stores both directions.
+  struct Pair {
+    int j, rk, back;  // the slot, its reverse slot and the residual there
+  };
+  __device__ __forceinline__ Pair pair(int, int j) const {
+    const int rk = rev[j];
+    return Pair{j, rk, dc[rk].y};
+  }
+  __device__ __forceinline__ void push_pair(const Pair &p, int res, int d) const {
+    dc[p.j].y = res - d;
+    dc[p.rk].y = p.back + d;
+    if (dirty) {
+      dirty[p.j >> 3] = 1;
+      dirty[p.rk >> 3] = 1;
+    }
+  }
   // BFS, two stages so a lane can keep several slots in flight:
   //   bfs_slot(j)   -> neighbour w of slot j and the index of the residual of the arc w -> u
   //   bfs_rin(idx)  -> that residual
@@ -99,6 +116,21 @@ struct LayoutBCSR2 {
     if (dirty) {
       dirty[key >> 3] = 1;
       dirty[rv >> 3] = 1;
+    }
+  }
+  struct Pair {
+    int j, rk, back;
+  };
+  __device__ __forceinline__ Pair pair(int, int j) const {
+    const int rk = cr[j].y;
+    return Pair{j, rk, cr[rk].x};
+  }
+  __device__ __forceinline__ void push_pair(const Pair &p, int res, int d) const {
+    cr[p.j].x = res - d;
+    cr[p.rk].x = p.back + d;
+    if (dirty) {
+      dirty[p.j >> 3] = 1;
+      dirty[p.rk >> 3] = 1;
     }
   }
   __device__ __forceinline__ void bfs_slot(int, int j, int &w, int &idx) const {
@@ -154,6 +186,17 @@ struct LayoutRCSR {
       atomicSub(&bcf[a], d);
       atomicAdd(&fdc[a].y, d);
     }
+  }
+  struct Pair {
+    int seg, a, back;  // the direction, the arc and the other direction's residual
+  };
+  __device__ __forceinline__ Pair pair(int seg, int j) const {
+    const int a = seg == 0 ? j : rdi[j].y;
+    return Pair{seg, a, seg == 0 ? bcf[a] : fdc[a].y};
+  }
+  __device__ __forceinline__ void push_pair(const Pair &p, int res, int d) const {
+    fdc[p.a].y = p.seg == 0 ? res - d : p.back + d;
+    bcf[p.a] = p.seg == 0 ? p.back + d : res - d;
   }
   __device__ __forceinline__ void bfs_slot(int seg, int j, int &w, int &idx) const {
     if (seg == 0) {  // forward arc u -> w: the arc w -> u is its backward direction

@@ -37,6 +37,7 @@
 #include "kernels.h"
 #include "mf_internal.h"
 #include "solver.h"
+#include "wg_launch.h"
 
 using namespace mfk;
 
@@ -2273,6 +2274,8 @@ static mf_status dmalloc(T **p, size_t count) {
   return MF_OK;
 }
 
+constexpr int kHubClass = 4;  // first degree class above 1,024 slots (class_config)
+
 static_assert(kClasses == kNumClasses, "host and device class counts differ");
 static_assert(kTunedClasses == sizeof(((mf_options *)nullptr)->class_lanes) / sizeof(uint16_t),
               "mf_options.class_lanes covers the tunable classes");
@@ -2368,6 +2371,8 @@ struct mf_context {
   void *staging = nullptr;  // pinned host buffer for packed batches (grown on demand)
   size_t staging_bytes = 0;
   bool cooperative = false;  // the device runs cooperative launches
+  int lds_limit = 0;         // LDS of one workgroup, bytes
+  mf::WgReport *wg_report = nullptr;  // host memory a one-workgroup solve writes its outcome to
 };
 
 namespace mf {
@@ -2419,6 +2424,7 @@ struct DevGraph {
   int64_t class_slots[kNumClasses] = {0};  // residual slots of the vertices of each VC class
   int64_t max_src_deg = 0;         // largest residual degree of a source
   int64_t giant_parts = 0;         // parts of all giants (kPartSlots slots each)
+  int64_t inner_hubs = 0;          // single graphs: vertices beside the terminals above 1,024 slots
   unsigned long long *giant = nullptr;  // per giant-list position: state of the parts
   // host copies for result read-back (single solves; batched uploads keep none)
   std::vector<int32_t> h_off, h_dst, h_cap, h_fslot, h_src, h_snk;
@@ -2521,6 +2527,10 @@ static mf_status set_vertex_classes(DevGraph &G, const std::vector<int64_t> &deg
     }
     G.giant_parts += pc[4 * kNumClasses];
   }
+  G.inner_hubs = G.vc_pop[kHubClass] + G.vc_pop[kHubClass + 1];
+  if (G.k == 1)
+    for (int32_t v : {G.h_src[0], G.h_snk[0]})
+      if (class_of_degree(vc, degree[(size_t)v]) >= kHubClass) --G.inner_hubs;
   // giant-list state, one entry per possible list position: no minimum, no parts, nothing
   // reserved (each giant's last part restores this)
   const size_t giants = (size_t)std::max<int64_t>(G.vc_pop[kNumClasses - 1], 1);
@@ -2699,9 +2709,114 @@ static mf_status upload(mf_context *ctx, const mf_csr *c, const int32_t *src, co
   return MF_OK;
 }
 
+// Residuals back to the capacities, unless no solve has run since the layout was built.
+static void restore_residuals(mf_context *ctx, DevGraph &G) {
+  if (G.fresh) return;
+  hipStream_t st = ctx->stream;
+  const int rgrid = std::max(1, (int)std::min<int64_t>((G.S + 255) / 256, 16 * ctx->num_cu));
+  if (G.dirty) {
+    const long long lines = (G.S + 7) / 8;
+    const int lgrid = std::max(1, (int)std::min<long long>((lines + 255) / 256, 16 * ctx->num_cu));
+    k_reset_dirty<<<lgrid, 256, 0, st>>>(G.layout == MF_LAYOUT_BCSR ? G.dc : G.cr, G.cap0, G.dirty,
+                                         lines, G.S, G.layout == MF_LAYOUT_BCSR ? 1 : 0);
+  } else {
+    if (G.layout == MF_LAYOUT_BCSR) k_reset_pairs<<<rgrid, 256, 0, st>>>(G.dc, G.cap0, G.S, 1);
+    else if (G.layout == MF_LAYOUT_BCSR2) k_reset_pairs<<<rgrid, 256, 0, st>>>(G.cr, G.cap0, G.S, 0);
+    else k_reset_pairs<<<rgrid, 256, 0, st>>>(G.fdc, G.cap0, G.m, 1);
+  }
+}
+
+// ---- single graphs inside one workgroup (wg_solve.h) ----
+//
+// Taken by graphs whose heights fit one CU's LDS, unless an option asks for a measurement or a
+// mechanism of the grid-wide kernels.  Tile widths, forwarding and BFS hand-over sizes tune those
+// kernels and have no meaning here.  Genrmf 16 x 16 x 16 10.5 -> 2.1 ms, Genrmf 29 x 29 x 47 55 -> 31
+// ms, a 64 x 64 random level graph 9.1 -> 1.7 ms, one of 8 x 8 0.82 -> 0.11 ms.
+//
+// Above kWgNarrowSlots residual slots only graphs without hubs (their levels scan as much as the
+// grid can take: R-MAT 15 would lose 1.2 ms before giving up, of 2.6), and only until a frontier of
+// the first global relabel holds more than kWgWide vertices: such levels and cycles have work for
+// the whole grid (matching of 8,000 + 8,000: 3.3 ms there, 4.1 ms here).
+constexpr int64_t kWgNarrowSlots = 1 << 15;
+constexpr int64_t kWgMaxSlots = 1 << 21;
+constexpr int kWgWide = 2048;
+
+static bool wg_allowed(const mf_options &o) {
+  return !o.verbose && !o.profile_kernels && !o.record_workload && !o.cycle_graphs &&
+         o.bfs_direction == 0;
+}
+
+// *taken: the solve is done (its status is returned); otherwise nothing has changed but the
+// residuals, which hold the capacities.
+template <class L>
+static mf_status run_one_workgroup(mf_context *ctx, DevGraph &G, const L &lay, const mf_options &o,
+                                   mf_result *res, bool *taken) {
+  *taken = false;
+  if (G.k != 1 || !wg_allowed(o) || G.S > kWgMaxSlots ||
+      (G.S > kWgNarrowSlots && G.inner_hubs > 0))
+    return MF_OK;
+  const int kind = wg_single_kind(G.n, ctx->lds_limit);
+  if (kind < 0) return MF_OK;
+  hipStream_t st = ctx->stream;
+  const double t0 = now_ms();
+  restore_residuals(ctx, G);
+  G.fresh = true;
+  const int rgrid = std::max(1, (int)std::min<int64_t>((G.S + 255) / 256, 16 * ctx->num_cu));
+  k_reset_vertices<<<rgrid, 256, 0, st>>>(G.h, G.e, G.stamp, G.n,
+                                          G.layout == MF_LAYOUT_RCSR ? G.bcf : nullptr, G.m);
+  HIP_TRY(hipGetLastError());
+  WgSingle a;
+  a.h = G.h;
+  a.e = G.e;
+  a.n = G.n;
+  a.s = G.h_src[0];
+  a.t = G.h_snk[0];
+  a.ratio = o.relabel_time_ratio > 0 ? o.relabel_time_ratio : kDefaultRelabelRatio;
+  if (o.cycles_per_relabel > 0) a.ratio = 1e30f;  // fixed cadence: only the count ends a round
+  a.max_cycles = o.cycles_per_relabel > 0 ? o.cycles_per_relabel : kMaxAdaptiveCycles;
+  a.max_rounds = o.max_rounds > 0 ? o.max_rounds : (int64_t)100000000;
+  a.wide = G.S > kWgNarrowSlots ? kWgWide : 0;
+  a.values = G.values;
+  a.report = ctx->wg_report;
+  a.lds_bytes = 0;
+  HIP_TRY(wg_single_launch(st, lay, a, kind, ctx->lds_limit));
+  HIP_TRY(hipStreamSynchronize(st));
+  const double t1 = now_ms();
+  const WgReport r = *ctx->wg_report;
+  if (r.status == 3) return MF_OK;
+  *taken = true;
+  G.fresh = false;
+  const mf_status status = r.status == 0 ? MF_OK
+                           : r.status == 1 ? MF_ERR_ITERATION_LIMIT : MF_ERR_INTERNAL;
+  if (res) {
+    memset(res, 0, sizeof(*res));
+    res->value = r.value;
+    res->source_outflow = r.source_out;
+    res->solve_ms = t1 - t0;
+    res->kernel_ms = (double)r.t_cycle * 1e-5;  // 100 MHz wall clock
+    res->relabel_ms = (double)r.t_relabel * 1e-5;
+    res->rounds = r.rounds;
+    res->cycles = r.cycles;
+    res->active_total = r.active;
+    res->slots_scanned = r.slots;
+    res->pushes = r.pushes;
+    res->relabels = r.relabels;
+    res->bfs_slots = r.bfs_slots;
+    res->bytes_algorithmic = algorithmic_bytes_cycle(G.layout, r.active, r.slots, r.pushes, r.relabels);
+    res->bytes_bfs = algorithmic_bytes_bfs(G.layout, G.n, r.rounds, r.bfs_verts, r.bfs_slots, 0, 0);
+    res->bfs_levels = r.levels;
+    res->status = status;
+  }
+  G.solved = (status == MF_OK);
+  return status;
+}
+
 template <class L>
 static mf_status run_solve(mf_context *ctx, DevGraph &G, const L &lay, mf_algo algo,
                            const mf_options &o, mf_result *res) {
+  bool taken = false;
+  const mf_status one = run_one_workgroup(ctx, G, lay, o, res, &taken);
+  if (taken || one != MF_OK) return one;
   hipStream_t st = ctx->stream;
   const int n = G.n;
   const ClassConfig cfg = class_config(algo, o.tile_lanes, o.class_lanes);
@@ -2881,17 +2996,7 @@ static mf_status run_solve(mf_context *ctx, DevGraph &G, const L &lay, mf_algo a
 
   const double t0 = now_ms();
   const int rgrid = std::max(1, (int)std::min<int64_t>((G.S + 255) / 256, 16 * ctx->num_cu));
-  // residuals back to the capacities, unless no solve has run since the layout was built
-  if (!G.fresh && G.dirty) {
-    const long long lines = (G.S + 7) / 8;
-    const int lgrid = std::max(1, (int)std::min<long long>((lines + 255) / 256, 16 * ctx->num_cu));
-    k_reset_dirty<<<lgrid, 256, 0, st>>>(G.layout == MF_LAYOUT_BCSR ? G.dc : G.cr, G.cap0, G.dirty,
-                                         lines, G.S, G.layout == MF_LAYOUT_BCSR ? 1 : 0);
-  } else if (!G.fresh) {
-    if (G.layout == MF_LAYOUT_BCSR) k_reset_pairs<<<rgrid, 256, 0, st>>>(G.dc, G.cap0, G.S, 1);
-    else if (G.layout == MF_LAYOUT_BCSR2) k_reset_pairs<<<rgrid, 256, 0, st>>>(G.cr, G.cap0, G.S, 0);
-    else k_reset_pairs<<<rgrid, 256, 0, st>>>(G.fdc, G.cap0, G.m, 1);
-  }
+  restore_residuals(ctx, G);
   G.fresh = false;
   k_reset_vertices<<<rgrid, 256, 0, st>>>(G.h, G.e, G.stamp, n,
                                           G.layout == MF_LAYOUT_RCSR ? G.bcf : nullptr,
@@ -3880,6 +3985,7 @@ mf_status mf_context_create(int device, mf_context **out) {
   mf_context *ctx = new mf_context();
   ctx->device = device;
   ctx->num_cu = prop.multiProcessorCount;
+  ctx->lds_limit = (int)prop.sharedMemPerBlock;
   int coop = 0;
   ctx->cooperative = hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, device) ==
                          hipSuccess &&
@@ -3890,7 +3996,9 @@ mf_status mf_context_create(int device, mf_context **out) {
       hipEventCreate(&ctx->ev_solve[0]) != hipSuccess ||
       hipEventCreate(&ctx->ev_solve[1]) != hipSuccess ||
       hipEventCreate(&ctx->ev_solve[2]) != hipSuccess ||
-      hipEventCreate(&ctx->ev_solve[3]) != hipSuccess) {
+      hipEventCreate(&ctx->ev_solve[3]) != hipSuccess ||
+      hipHostMalloc((void **)&ctx->wg_report, sizeof(WgReport),
+                    hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess) {
     mf_context_destroy(ctx);
     return MF_ERR_DEVICE;
   }
@@ -3910,6 +4018,7 @@ mf_status mf_context_destroy(mf_context *ctx) {
   for (hipEvent_t e : ctx->ev_solve)
     if (e) (void)hipEventDestroy(e);
   if (ctx->staging) (void)hipHostFree(ctx->staging);
+  if (ctx->wg_report) (void)hipHostFree(ctx->wg_report);
   if (ctx->stream) (void)hipStreamDestroy(ctx->stream);
   delete ctx;
   return MF_OK;
