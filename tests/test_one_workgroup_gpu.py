@@ -56,7 +56,8 @@ def check(mf, orc, ctx, g):
     (1301, 20),    # more: excesses in global memory
     (1500, 41),    # nearly as many as fit at all
     (1600, 42),    # too many
-    (2048, 9), (2049, 9),  # the widest frontier that stays, and one more vertex
+    (2048, 13), (2049, 13),  # the widest frontiers that stay with excesses in global memory, and wider
+    (2800, 8), (2801, 8), (4000, 2),  # and in LDS; two wide frontiers stay
 ])
 def test_chains(mf, orc, ctx, width, length):
     check(mf, orc, ctx, chains(mf, width, length, seed=width + length))

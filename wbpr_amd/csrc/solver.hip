@@ -2372,7 +2372,6 @@ struct mf_context {
   size_t staging_bytes = 0;
   bool cooperative = false;  // the device runs cooperative launches
   int lds_limit = 0;         // LDS of one workgroup, bytes
-  mf::WgReport *wg_report = nullptr;  // host memory a one-workgroup solve writes its outcome to
 };
 
 namespace mf {
@@ -2733,13 +2732,17 @@ static void restore_residuals(mf_context *ctx, DevGraph &G) {
 // kernels and have no meaning here.  Genrmf 16 x 16 x 16 10.5 -> 2.1 ms, Genrmf 29 x 29 x 47 55 -> 31
 // ms, a 64 x 64 random level graph 9.1 -> 1.7 ms, one of 8 x 8 0.82 -> 0.11 ms.
 //
-// Above kWgNarrowSlots residual slots only graphs without hubs (their levels scan as much as the
-// grid can take: R-MAT 15 would lose 1.2 ms before giving up, of 2.6), and only until a frontier of
-// the first global relabel holds more than kWgWide vertices: such levels and cycles have work for
-// the whole grid (matching of 8,000 + 8,000: 3.3 ms there, 4.1 ms here).
+// Above kWgNarrowSlots residual slots only graphs without hubs, whose levels scan as much as the
+// grid can take (R-MAT 13, edge factor 8: 0.92 ms there, 1.8 ms here), and only with frontiers that
+// are narrow next to the workgroup, seen in the first global relabel.  With the excesses in LDS too a
+// graph may have kWgWideLevels wide ones -- a matching network has two, and is still solved
+// sooner here: 8,000 + 8,000 vertices 3.8 ms there, 1.6 ms here -- before it counts as wide and
+// deep, work for the whole grid; with the excesses in global memory none (16,000 + 16,000: 3.9 and
+// 3.2 ms, 20,000 + 20,500: 2.3 and 2.8 ms, Genrmf 48 x 48 x 20: 32 and 40 ms).
 constexpr int64_t kWgNarrowSlots = 1 << 15;
 constexpr int64_t kWgMaxSlots = 1 << 21;
-constexpr int kWgWide = 2048;
+constexpr int kWgWideBoth = 2800, kWgWideHeights = 2048;
+constexpr int kWgWideLevels = 2;
 
 static bool wg_allowed(const mf_options &o) {
   return !o.verbose && !o.profile_kernels && !o.record_workload && !o.cycle_graphs &&
@@ -2775,14 +2778,18 @@ static mf_status run_one_workgroup(mf_context *ctx, DevGraph &G, const L &lay, c
   if (o.cycles_per_relabel > 0) a.ratio = 1e30f;  // fixed cadence: only the count ends a round
   a.max_cycles = o.cycles_per_relabel > 0 ? o.cycles_per_relabel : kMaxAdaptiveCycles;
   a.max_rounds = o.max_rounds > 0 ? o.max_rounds : (int64_t)100000000;
-  a.wide = G.S > kWgNarrowSlots ? kWgWide : 0;
+  const bool both = kind == kWgBoth;
+  a.wide = G.S > kWgNarrowSlots ? (both ? kWgWideBoth : kWgWideHeights) : 0;
+  a.wide_levels = both ? kWgWideLevels : 0;
   a.values = G.values;
-  a.report = ctx->wg_report;
+  static_assert(sizeof(WgReport) <= sizeof(int) * CTL_SIZE, "the report fits the control words");
+  a.report = reinterpret_cast<WgReport *>(G.ctl);  // the grid-wide kernels' words, free here
   a.lds_bytes = 0;
   HIP_TRY(wg_single_launch(st, lay, a, kind, ctx->lds_limit));
+  WgReport r;
+  HIP_TRY(hipMemcpyAsync(&r, G.ctl, sizeof(r), hipMemcpyDeviceToHost, st));
   HIP_TRY(hipStreamSynchronize(st));
   const double t1 = now_ms();
-  const WgReport r = *ctx->wg_report;
   if (r.status == 3) return MF_OK;
   *taken = true;
   G.fresh = false;
@@ -3371,15 +3378,29 @@ static mf_status run_batch_wg(mf_context *ctx, DevGraph &G, const int32_t *vbase
   const int32_t k = G.k;
   const ClassConfig vc = class_config(MF_ALGO_VC, 0);
   const ClassConfig cc = class_config(algo, o.tile_lanes, o.class_lanes);
-  // class populations of every instance, from the slot degrees upload() recorded (the same
+  std::vector<int32_t> nver((size_t)k), order((size_t)k);
+  for (int32_t i = 0; i < k; ++i) {
+    nver[(size_t)i] = vbase[i + 1] - vbase[i];
+    order[(size_t)i] = i;
+  }
+  std::stable_sort(order.begin(), order.end(),
+                   [&](int32_t x, int32_t y) { return nver[(size_t)x] > nver[(size_t)y]; });
+  // Largest first: [0, huge) too large for the LDS kernels, [huge, large) with a CU each, the rest
+  // four to a CU -- unless there are CUs for all: an instance is solved soonest with a whole one.
+  int32_t huge = 0;
+  while (huge < k && !wg_batch_takes(nver[(size_t)order[(size_t)huge]], ctx->lds_limit)) ++huge;
+  int32_t large = huge;
+  while (large < k && (k - huge <= ctx->num_cu ||
+                       nver[(size_t)order[(size_t)large]] > kWgSmallVertices))
+    ++large;
+  // class populations of the huge instances, from the slot degrees upload() recorded (the same
   // classes it stored on the device)
-  std::vector<int32_t> nver((size_t)k), pop((size_t)k * kNumClasses, 0),
-      bpop((size_t)k * kNumClasses, 0), order((size_t)k);
+  std::vector<int32_t> pop((size_t)k * kNumClasses, 0), bpop((size_t)k * kNumClasses, 0);
   parallel_for(
-      k,
+      huge,
       [&](int64_t b, int64_t e) {
-        for (int64_t i = b; i < e; ++i) {
-          nver[(size_t)i] = vbase[i + 1] - vbase[i];
+        for (int64_t q = b; q < e; ++q) {
+          const int32_t i = order[(size_t)q];
           for (int32_t v = vbase[i]; v < vbase[i + 1]; ++v) {
             const int64_t deg = G.degree[(size_t)v];
             bpop[(size_t)i * kNumClasses + class_of_degree(vc, deg)]++;
@@ -3388,9 +3409,6 @@ static mf_status run_batch_wg(mf_context *ctx, DevGraph &G, const int32_t *vbase
         }
       },
       1);
-  for (int32_t i = 0; i < k; ++i) order[(size_t)i] = i;
-  std::stable_sort(order.begin(), order.end(),
-                   [&](int32_t x, int32_t y) { return nver[(size_t)x] > nver[(size_t)y]; });
   int *d_vbase = nullptr, *d_nver = nullptr, *d_pop = nullptr, *d_bpop = nullptr,
       *d_order = nullptr, *d_next = nullptr, *d_status = nullptr;
   auto cleanup = [&]() {
@@ -3402,15 +3420,16 @@ static mf_status run_batch_wg(mf_context *ctx, DevGraph &G, const int32_t *vbase
   if ((rc = dmalloc(&d_vbase, (size_t)k)) || (rc = dmalloc(&d_nver, (size_t)k)) ||
       (rc = dmalloc(&d_pop, (size_t)k * kNumClasses)) ||
       (rc = dmalloc(&d_bpop, (size_t)k * kNumClasses)) || (rc = dmalloc(&d_order, (size_t)k)) ||
-      (rc = dmalloc(&d_next, (size_t)1)) || (rc = dmalloc(&d_status, (size_t)k))) {
+      (rc = dmalloc(&d_next, (size_t)3)) || (rc = dmalloc(&d_status, (size_t)k))) {
     cleanup();
     return rc;
   }
   bool ok =
       hipMemcpyAsync(d_vbase, vbase, sizeof(int) * k, hipMemcpyHostToDevice, st) == hipSuccess &&
       hipMemcpyAsync(d_nver, nver.data(), sizeof(int) * k, hipMemcpyHostToDevice, st) == hipSuccess &&
-      hipMemcpyAsync(d_pop, pop.data(), sizeof(int) * pop.size(), hipMemcpyHostToDevice, st) == hipSuccess &&
-      hipMemcpyAsync(d_bpop, bpop.data(), sizeof(int) * bpop.size(), hipMemcpyHostToDevice, st) == hipSuccess &&
+      (huge == 0 ||
+       (hipMemcpyAsync(d_pop, pop.data(), sizeof(int) * pop.size(), hipMemcpyHostToDevice, st) == hipSuccess &&
+        hipMemcpyAsync(d_bpop, bpop.data(), sizeof(int) * bpop.size(), hipMemcpyHostToDevice, st) == hipSuccess)) &&
       hipMemcpyAsync(d_order, order.data(), sizeof(int) * k, hipMemcpyHostToDevice, st) == hipSuccess &&
       hipStreamSynchronize(st) == hipSuccess;
   if (!ok) {
@@ -3431,7 +3450,7 @@ static mf_status run_batch_wg(mf_context *ctx, DevGraph &G, const int32_t *vbase
   b.bpop = d_bpop;
   b.vcls = G.vcls;
   b.order = d_order;
-  b.k = k;
+  b.k = huge;
   b.next = d_next;
   b.values = G.values;
   b.status = d_status;
@@ -3449,14 +3468,23 @@ static mf_status run_batch_wg(mf_context *ctx, DevGraph &G, const int32_t *vbase
   b.fwd_hops = o.forward_hops < 0 ? 0 : (o.forward_hops > 0 ? o.forward_hops : kDefaultForwardHops);
   b.stamp = G.stamp;
   if (o.cycles_per_relabel > 0) b.ratio = 1e30f;  // fixed cadence: only the cycle cap ends a round
-  // persistent workgroups: as many as can be resident at once (the kernel's registers decide),
-  // so none waits for another to finish before it starts pulling instances
-  int per_cu = 0;
-  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_batch_wg<LayoutBCSR>, kBlock, 0) !=
-          hipSuccess ||
-      per_cu < 1)
-    per_cu = 1;
-  const int nwg = std::max(1, std::min(k, std::min(per_cu, kBatchGroupsPerCU) * ctx->num_cu));
+  WgBatch w;
+  w.h = G.h;
+  w.e = G.e;
+  w.vbase = d_vbase;
+  w.nver = d_nver;
+  w.src = G.src;
+  w.snk = G.snk;
+  w.order = d_order + huge;
+  w.k = k - huge;
+  w.next = d_next + 1;
+  w.values = G.values;
+  w.status = d_status;
+  w.stats = G.stats;
+  w.ratio = b.ratio;
+  w.max_cycles = b.max_cycles;
+  w.max_rounds = b.max_rounds;
+  w.lds_bytes = 0;
   const double t0 = now_ms();
   const int rgrid = std::max(1, (int)std::min<int64_t>((G.S + 255) / 256, 16 * ctx->num_cu));
   if (!G.fresh) k_reset_pairs<<<rgrid, 256, 0, st>>>(G.dc, G.cap0, G.S, 1);
@@ -3464,11 +3492,27 @@ static mf_status run_batch_wg(mf_context *ctx, DevGraph &G, const int32_t *vbase
   k_reset_vertices<<<rgrid, 256, 0, st>>>(G.h, G.e, G.stamp, G.n, nullptr, 0);
   if (hipMemsetAsync(G.stats, 0, sizeof(unsigned long long) * kStatSlot * kStatSpread, st) != hipSuccess ||
       hipMemsetAsync(G.ctl, 0, sizeof(int) * CTL_SIZE, st) != hipSuccess ||
-      hipMemsetAsync(d_next, 0, sizeof(int), st) != hipSuccess) {
+      hipMemsetAsync(d_next, 0, 3 * sizeof(int), st) != hipSuccess) {
     cleanup();
     return MF_ERR_DEVICE;
   }
-  k_batch_wg<LayoutBCSR><<<nwg, kBlock, 0, st>>>(G.bcsr(), b);
+  if (huge > 0) {
+    // persistent workgroups: as many as can be resident at once (the kernel's registers decide),
+    // so none waits for another to finish before it starts pulling instances
+    int per_cu = 0;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_batch_wg<LayoutBCSR>, kBlock, 0) !=
+            hipSuccess ||
+        per_cu < 1)
+      per_cu = 1;
+    const int nwg = std::min(huge, std::min(per_cu, kBatchGroupsPerCU) * ctx->num_cu);
+    k_batch_wg<LayoutBCSR><<<nwg, kBlock, 0, st>>>(G.bcsr(), b);
+  }
+  if (huge < k && wg_batch_launch(st, G.bcsr(), w, large - huge, ctx->num_cu, ctx->lds_limit) !=
+                      hipSuccess) {
+    (void)hipStreamSynchronize(st);
+    cleanup();
+    return MF_ERR_DEVICE;
+  }
   std::vector<int> status((size_t)k);
   unsigned long long hs[kStatSlot];
   int hctl[CTL_SIZE];
@@ -3996,9 +4040,7 @@ mf_status mf_context_create(int device, mf_context **out) {
       hipEventCreate(&ctx->ev_solve[0]) != hipSuccess ||
       hipEventCreate(&ctx->ev_solve[1]) != hipSuccess ||
       hipEventCreate(&ctx->ev_solve[2]) != hipSuccess ||
-      hipEventCreate(&ctx->ev_solve[3]) != hipSuccess ||
-      hipHostMalloc((void **)&ctx->wg_report, sizeof(WgReport),
-                    hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess) {
+      hipEventCreate(&ctx->ev_solve[3]) != hipSuccess) {
     mf_context_destroy(ctx);
     return MF_ERR_DEVICE;
   }
@@ -4018,7 +4060,6 @@ mf_status mf_context_destroy(mf_context *ctx) {
   for (hipEvent_t e : ctx->ev_solve)
     if (e) (void)hipEventDestroy(e);
   if (ctx->staging) (void)hipHostFree(ctx->staging);
-  if (ctx->wg_report) (void)hipHostFree(ctx->wg_report);
   if (ctx->stream) (void)hipStreamDestroy(ctx->stream);
   delete ctx;
   return MF_OK;

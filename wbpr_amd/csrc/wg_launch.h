@@ -5,9 +5,15 @@
 
 #include <cstdint>
 
+#include "kernels.h"
+
+namespace mfk {
+enum WgKind { kWgBoth = 0, kWgHeights = 1, kWgGlobal = 2 };  // see wg_solve.h
+}
+
 namespace mf {
 
-// What a solve did, written by its kernel into host memory.
+// What a solve did.
 struct WgReport {
   long long value;
   int status;  // WgOutcome::status
@@ -22,18 +28,46 @@ struct WgSingle {
   float ratio;         // cycle time / relabel time per round
   int max_cycles;      // cycles per round
   long long max_rounds;
-  int wide;            // > 0: give up when a frontier of the first relabel is wider
+  int wide;            // > 0: give up when more than wide_levels frontiers of the first relabel
+  int wide_levels;     // hold more vertices than this
   long long *values;   // [0] receives the value
-  WgReport *report;    // host memory the device writes
+  WgReport *report;    // device memory
   int lds_bytes;       // (set by the launch)
 };
 
 constexpr int kWgStaticLds = 4096;  // LDS kept back for the kernels' static arrays
-constexpr int kWgMinList = 2048;    // list entries an instance's LDS has room for at least
 
 // How a graph of n vertices is held (a WgKind), or -1: its state does not fit lds_limit.
 int wg_single_kind(int32_t n, int lds_limit);
 template <class L>
 hipError_t wg_single_launch(hipStream_t st, const L &g, WgSingle a, int kind, int lds_limit);
+
+// A batch: every instance of order[0, k) inside one workgroup of a persistent grid.
+struct WgBatch {
+  int *h, *e;            // global arrays over all vertices; the excesses must be zero
+  const int *vbase, *nver, *src, *snk;
+  const int *order;      // instances, largest first
+  int k;
+  int *next;             // queue heads of the launches, zero
+  long long *values;
+  int *status;           // per instance: WgOutcome::status
+  unsigned long long *stats;
+  float ratio;
+  int max_cycles;
+  long long max_rounds;
+  int lds_bytes;         // (set by the launch)
+};
+
+// Instances of more vertices take kWgThreads threads and a CU's whole LDS each; the others
+// kWgSmallThreads and a quarter of it, four to a CU.
+constexpr int kWgSmallVertices = 4096;
+
+// Whether the batch kernels take an instance of n vertices.
+bool wg_batch_takes(int32_t n, int lds_limit);
+// Instances order[0, large) with a CU each, then order[large, k) four to a CU.  Largest first: the
+// first launch ends on its smallest instances, so the second need not overlap it.  a.next: two
+// words.
+hipError_t wg_batch_launch(hipStream_t st, const mfk::LayoutBCSR &g, WgBatch a, int large,
+                           int num_cu, int lds_limit);
 
 }  // namespace mf

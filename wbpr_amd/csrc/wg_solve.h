@@ -10,36 +10,51 @@
 // Kinds of instance (WgKind), by what fits one CU's 160 KB of LDS:
 //   kWgBoth     heights (16 bits: at most n + 1) and excesses (32 bits) in LDS, up to about 24,700
 //               vertices;
-//   kWgHeights  heights in LDS, excesses in global memory, up to about 63,000 vertices.
+//   kWgHeights  heights in LDS, excesses in global memory, up to about 63,000 vertices;
+//   kWgGlobal   both in global memory, up to kWgMaxVertices (batched instances: a single graph of
+//               that size has the whole grid).
 // The rest of the LDS holds two vertex lists (BFS frontiers, then cycle worklists).  A list that
 // outgrows its part loses nothing: the next level or cycle finds its vertices by their height or
 // excess instead of by the list.
 #pragma once
 
+#include <type_traits>
+
 #include "kernels.h"
+#include "wg_launch.h"
 
 namespace mfk {
 
-enum WgKind { kWgBoth = 0, kWgHeights = 1 };
-
 constexpr int kWgThreads = 1024;      // workgroup of the instances that fill a CU's LDS
 constexpr int kWgMaxHeights = 65533;  // vertices whose heights (0 .. n + 1) fit 16 bits
+constexpr int kWgMaxVertices = 1 << 19;  // the bitmap alone takes 64 KB of LDS then
 // Vertices of more residual slots than this are discharged by a whole wave, and expanded by the
 // whole workgroup in the BFS; the others by tiles of 8 or 2 lanes.
 constexpr int kWgHubSlots = 96;
 constexpr int kWgHubCap = 256;        // hubs waiting at a time; the others stay in the worklist
+constexpr int kWgMinList = 2048;      // list entries an instance's LDS has room for at least
 constexpr int kWgClockMask = 7;       // the clock is read every 8th cycle
-// kWgHeights: entries of the table that sums a pass's pushes by target (at most one push per
+// kWgHeights, kWgGlobal: entries of the table that sums a pass's pushes by target (at most one push per
 // 2-lane tile, so at most a quarter full)
 constexpr int kWgTable = 2048;
 
 __host__ __device__ constexpr int wg_bits_words(int n) { return (n + 63) / 64 * 2; }
 // LDS bytes of an instance's vertex state without the lists
 __host__ __device__ constexpr long long wg_state_bytes(int kind, long long n) {
-  return (kind == kWgBoth ? 4 * n : 8 * kWgTable) + (2 * n + 3) / 4 * 4 +
+  return (kind == kWgBoth ? 4 * n : 8 * kWgTable) + (kind == kWgGlobal ? 0 : (2 * n + 3) / 4 * 4) +
          4LL * wg_bits_words((int)n);
 }
-constexpr int kWgItemBytes = 2;  // a list entry: a local vertex id
+// bytes of a list entry: a local vertex id
+__host__ __device__ constexpr int wg_item_bytes(int kind) { return kind == kWgGlobal ? 4 : 2; }
+// The kind of an instance of n vertices in `room` bytes of LDS, or -1.
+__host__ __device__ constexpr int wg_kind(long long n, long long room) {
+  for (int kind = kWgBoth; kind <= kWgGlobal; ++kind) {
+    if (n > (kind == kWgGlobal ? kWgMaxVertices : kWgMaxHeights)) continue;
+    const long long items = n < kWgMinList ? n : kWgMinList;
+    if (wg_state_bytes(kind, n) + 2 * wg_item_bytes(kind) * items <= room) return kind;
+  }
+  return -1;
+}
 
 struct WgShared {
   int cnt[3];   // items of the list a cycle or level reads (q % 3), fills ((q + 1) % 3), clears
@@ -75,7 +90,11 @@ __device__ __forceinline__ unsigned tile_minu(unsigned v) {
 
 template <class L, int KIND, int BS>
 struct WgSolver {
-  using HT = unsigned short;  // heights, list entries
+  // heights and list entries; a lane's lowest (height, slot)
+  using HT = typename std::conditional<KIND == kWgGlobal, int, unsigned short>::type;
+  using Key = typename std::conditional<KIND == kWgGlobal, unsigned long long, unsigned>::type;
+  static constexpr int kSlotBits = KIND == kWgGlobal ? 32 : 16;
+  static constexpr Key kNone = ~(Key)0;
 
   const L &g;
   WgShared &S;
@@ -84,7 +103,7 @@ struct WgSolver {
   int *e;           // excesses, local ids
   unsigned *bits;   // BFS: reached; an overflowed worklist: its vertices
   HT *lists;        // two lists of cap entries
-  int *tkey, *tsum; // kWgHeights: the table of a pass's pushes (key -1: empty)
+  int *tkey, *tsum; // kWgHeights, kWgGlobal: the table of a pass's pushes (key -1: empty)
   int cap;
   WgStats st;
 
@@ -107,7 +126,7 @@ struct WgSolver {
   }
 
   // Divides the dynamic LDS among the state arrays; the lists take what is left.
-  __device__ __forceinline__ void carve(char *lds, int lds_bytes, int *ge) {
+  __device__ __forceinline__ void carve(char *lds, int lds_bytes, int *gh, int *ge) {
     char *p = lds;
     if constexpr (KIND == kWgBoth) {
       e = reinterpret_cast<int *>(p);
@@ -120,9 +139,13 @@ struct WgSolver {
     }
     bits = reinterpret_cast<unsigned *>(p);
     p += 4 * wg_bits_words(n);
-    h = reinterpret_cast<HT *>(p);
-    p += (2 * n + 3) / 4 * 4;
-    cap = min(n, (int)((lds + lds_bytes - p) / (2 * kWgItemBytes)));
+    if constexpr (KIND == kWgGlobal) {
+      h = reinterpret_cast<HT *>(gh + vb);
+    } else {
+      h = reinterpret_cast<HT *>(p);
+      p += (2 * n + 3) / 4 * 4;
+    }
+    cap = min(n, (int)((lds + lds_bytes - p) / (2 * wg_item_bytes(KIND))));
     lists = reinterpret_cast<HT *>(p);
   }
   // (an array of two pointers, indexed at run time, would put the whole object in scratch memory)
@@ -190,7 +213,7 @@ struct WgSolver {
         if (lane == 0) defer(u, hubs, nhub, out, ocnt);
         go = false;
       }
-      unsigned best = ~0u;
+      Key best = kNone;
       int bw = 0, bres = 0;
       if (go) {
         for (int x0 = lane; x0 < r.d; x0 += T * B) {
@@ -201,11 +224,11 @@ struct WgSolver {
             int key;
             g.scan(r.seg(x), r.at(x), w[b], res[b], key);
           }
-          unsigned k[B];
+          Key k[B];
 #pragma unroll
           for (int b = 0; b < B; ++b) {
             w[b] -= vb;
-            k[b] = ((unsigned)h[w[b]] << 16) | (unsigned)(x0 + b * T);
+            k[b] = ((Key)(unsigned)h[w[b]] << kSlotBits) | (unsigned)(x0 + b * T);
           }
 #pragma unroll
           for (int b = 0; b < B; ++b) {
@@ -217,14 +240,16 @@ struct WgSolver {
           }
         }
       }
-      const unsigned low = tile_minu<T>(best);
-      const int hmin = (int)(low >> 16);
-      const bool dead = low == ~0u || hmin + 1 >= n;
+      Key low;
+      if constexpr (KIND == kWgGlobal) low = tile_min<T>(best);
+      else low = tile_minu<T>(best);
+      const int hmin = (int)(low >> kSlotBits);
+      const bool dead = low == kNone || hmin + 1 >= n;
       const int hnew = dead ? n : max(hu, hmin + 1);
       const bool winner = go && !dead && best == low;  // one lane: keys are unique
       typename L::Pair pair;
       if (winner) {
-        const int x = (int)(best & 0xffffu);
+        const int x = (int)(best & (((Key)1 << kSlotBits) - 1));
         pair = g.pair(r.seg(x), r.at(x));
       }
       if (go && lane == 0) {
@@ -265,7 +290,7 @@ struct WgSolver {
     }
   }
 
-  // kWgHeights: d more for w in this pass.  Excesses in global memory take no atomics (see above):
+  // kWgHeights, kWgGlobal: d more for w in this pass.  Excesses in global memory take no atomics (see above):
   // a pass's pushes are summed by target here, and the lane whose push made the entry, which gets
   // its index (the others -1), adds the sum to e(w) behind the next barrier.
   __device__ __forceinline__ int table_add(int w, int d) {
@@ -456,9 +481,9 @@ struct WgSolver {
   }
 
   // Heights from a BFS over reverse residual arcs: distances to the sink, n where it cannot be
-  // reached.  Returns the levels; wide > 0 gives up (-1) at the first frontier of more vertices
-  // than that, before anything outside LDS has been written.
-  __device__ __forceinline__ int relabel(int wide, bool check) {
+  // reached.  Returns the levels; wide > 0 gives up (-1) once more than wide_levels frontiers held
+  // more vertices than that, before anything outside LDS has been written.
+  __device__ __forceinline__ int relabel(int wide, int wide_levels, bool check) {
     const int tid = (int)threadIdx.x;
     for (int v = tid; v < n; v += BS) h[v] = (HT)(v == s ? n + 1 : (v == t ? 0 : n));
     for (int w = tid; w < wg_bits_words(n); w += BS) {
@@ -480,7 +505,7 @@ struct WgSolver {
     for (;; ++level) {
       const int cnt = S.cnt[level % 3];
       if (cnt == 0) break;
-      if (wide > 0 && cnt > wide) return -1;
+      if (wide > 0 && cnt > wide && wide_levels-- == 0) return -1;
       if (tid == 0) {
         S.cnt[(level + 2) % 3] = 0;
         // (filled in the level that uses it, and read after that level's barrier: the next level's
@@ -519,7 +544,7 @@ struct WgSolver {
   // The residuals hold the capacities and every excess is zero on entry.  Every thread of the
   // workgroup calls this and returns the same outcome (source_out aside).
   __device__ __forceinline__ WgOutcome solve(float ratio, int max_cycles, long long max_rounds,
-                                             int wide) {
+                                             int wide, int wide_levels) {
     const int tid = (int)threadIdx.x;
     WgOutcome o{0, 0, 0, 0, 0, 0, 0, 0};
     if constexpr (KIND == kWgBoth) {
@@ -536,7 +561,7 @@ struct WgSolver {
         break;
       }
       const long long t0 = (long long)wall_clock64();
-      const int levels = relabel(round == 0 ? wide : 0, round > 0);
+      const int levels = relabel(round == 0 ? wide : 0, wide_levels, round > 0);
       if (levels < 0) {
         o.status = 3;
         break;

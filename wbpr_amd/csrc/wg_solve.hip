@@ -10,7 +10,7 @@ using namespace mfk;
 
 namespace mf {
 
-// Sums over the workgroup into the report (host memory), by its first thread.
+// Sums over the workgroup into the report, by its first thread.
 __device__ __forceinline__ void write_report(WgReport *rep, const WgOutcome &o, const WgStats &st) {
   __shared__ unsigned long long tot[7];
   if (threadIdx.x < 7) tot[threadIdx.x] = 0;
@@ -48,8 +48,8 @@ __global__ __launch_bounds__(kWgThreads) void k_wg_solve(L g, WgSingle a) {
   __shared__ WgShared S;
   WgSolver<L, KIND, kWgThreads> w{g, S, 0, a.n, a.s, a.t};
   w.st = WgStats{0, 0, 0, 0, 0, 0};
-  w.carve(lds, a.lds_bytes, a.e);
-  const WgOutcome o = w.solve(a.ratio, a.max_cycles, a.max_rounds, a.wide);
+  w.carve(lds, a.lds_bytes, a.h, a.e);
+  const WgOutcome o = w.solve(a.ratio, a.max_cycles, a.max_rounds, a.wide, a.wide_levels);
   if (o.status != 3) {
     for (int v = (int)threadIdx.x; v < a.n; v += kWgThreads) {
       a.h[v] = w.h[v];
@@ -61,13 +61,8 @@ __global__ __launch_bounds__(kWgThreads) void k_wg_solve(L g, WgSingle a) {
 }
 
 int wg_single_kind(int32_t n, int lds_limit) {
-  const long long room = (long long)lds_limit - kWgStaticLds;
-  for (int kind : {(int)kWgBoth, (int)kWgHeights}) {
-    if (n > kWgMaxHeights) continue;
-    const long long lists = 2LL * kWgItemBytes * std::min<int32_t>(n, kWgMinList);
-    if (wg_state_bytes(kind, n) + lists <= room) return kind;
-  }
-  return -1;
+  const int kind = wg_kind(n, (long long)lds_limit - kWgStaticLds);
+  return kind == kWgGlobal ? -1 : kind;
 }
 
 template <class L, int KIND>
@@ -82,7 +77,7 @@ static hipError_t launch_single(hipStream_t st, const L &g, const WgSingle &a) {
 
 template <class L>
 hipError_t wg_single_launch(hipStream_t st, const L &g, WgSingle a, int kind, int lds_limit) {
-  const long long all = wg_state_bytes(kind, a.n) + 2LL * kWgItemBytes * a.n;
+  const long long all = wg_state_bytes(kind, a.n) + 2LL * wg_item_bytes(kind) * a.n;
   a.lds_bytes = (int)std::min<long long>((all + 15) / 16 * 16, lds_limit - kWgStaticLds);
   return kind == kWgBoth ? launch_single<L, kWgBoth>(st, g, a)
                          : launch_single<L, kWgHeights>(st, g, a);
@@ -90,5 +85,79 @@ hipError_t wg_single_launch(hipStream_t st, const L &g, WgSingle a, int kind, in
 template hipError_t wg_single_launch(hipStream_t, const LayoutBCSR &, WgSingle, int, int);
 template hipError_t wg_single_launch(hipStream_t, const LayoutBCSR2 &, WgSingle, int, int);
 template hipError_t wg_single_launch(hipStream_t, const LayoutRCSR &, WgSingle, int, int);
+
+// ---- batches ----
+
+constexpr int kWgSmallThreads = 256;
+static_assert(wg_state_bytes(kWgBoth, kWgSmallVertices) + 4LL * kWgMinList <=
+                  163840 / 4 - kWgStaticLds,
+              "a small instance fits a quarter of 160 KB with its excesses");
+
+template <int KIND, int BS>
+__device__ __forceinline__ void batch_one(const LayoutBCSR &g, const WgBatch &a, char *lds,
+                                          WgShared &S, int inst) {
+  const int vb = a.vbase[inst];
+  WgSolver<LayoutBCSR, KIND, BS> w{g, S, vb, a.nver[inst], a.src[inst] - vb, a.snk[inst] - vb};
+  w.st = WgStats{0, 0, 0, 0, 0, 0};
+  w.carve(lds, a.lds_bytes, a.h, a.e);
+  const WgOutcome o = w.solve(a.ratio, a.max_cycles, a.max_rounds, 0, 0);
+  if (threadIdx.x == 0) {
+    a.values[inst] = o.value;
+    a.status[inst] = o.status;
+  }
+  block_flush(w.st.active, w.st.slots, w.st.pushes, w.st.relabels, a.stats, ST_ACTIVE);
+  block_flush(w.st.bfs_verts, w.st.bfs_slots, 0, 0, a.stats, ST_BFS_VERTS);
+}
+
+template <int BS>
+__global__ __launch_bounds__(BS) void k_wg_batch(LayoutBCSR g, WgBatch a) {
+  extern __shared__ __align__(16) char lds[];
+  __shared__ WgShared S;
+  __shared__ int s_next;
+  for (;;) {
+    if (threadIdx.x == 0) s_next = atomicAdd(a.next, 1);
+    __syncthreads();
+    const int i = s_next;
+    __syncthreads();
+    if (i >= a.k) break;
+    const int inst = a.order[i];
+    const int kind = BS == kWgSmallThreads ? (int)kWgBoth : wg_kind(a.nver[inst], a.lds_bytes);
+    if (kind == kWgBoth) batch_one<kWgBoth, BS>(g, a, lds, S, inst);
+    else if (kind == kWgHeights) batch_one<kWgHeights, BS>(g, a, lds, S, inst);
+    else batch_one<kWgGlobal, BS>(g, a, lds, S, inst);
+  }
+}
+
+bool wg_batch_takes(int32_t n, int lds_limit) {
+  return wg_kind(n, (long long)lds_limit - kWgStaticLds) >= 0;
+}
+
+template <int BS>
+static hipError_t launch_batch(hipStream_t st, const LayoutBCSR &g, const WgBatch &a, int grid) {
+  const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(k_wg_batch<BS>),
+                                           hipFuncAttributeMaxDynamicSharedMemorySize, a.lds_bytes);
+  if (e != hipSuccess) return e;
+  k_wg_batch<BS><<<grid, BS, a.lds_bytes, st>>>(g, a);
+  return hipGetLastError();
+}
+
+hipError_t wg_batch_launch(hipStream_t st, const LayoutBCSR &g, WgBatch a, int large, int num_cu,
+                           int lds_limit) {
+  const int k = a.k;
+  hipError_t e = hipSuccess;
+  if (large > 0) {
+    a.k = large;
+    a.lds_bytes = (lds_limit - kWgStaticLds) & ~15;
+    e = launch_batch<kWgThreads>(st, g, a, std::min(large, num_cu));
+  }
+  if (e == hipSuccess && k > large) {
+    a.order += large;
+    a.k = k - large;
+    a.next += 1;
+    a.lds_bytes = (lds_limit / 4 - kWgStaticLds) & ~15;
+    e = launch_batch<kWgSmallThreads>(st, g, a, std::min(k - large, 4 * num_cu));
+  }
+  return e;
+}
 
 }  // namespace mf
