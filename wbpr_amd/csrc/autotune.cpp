@@ -283,7 +283,8 @@ mf_status mf_batch_autotune(mf_context *ctx, const mf_csr *inst, int32_t k, int3
   o.profile_kernels = 0;
   // the sample is packed and uploaded once; every trial solves it from the capacities again
   mf::PackedBatch packed;
-  mf_status pst = mf::pack_instances(ctx, sub.data(), (int32_t)sub.size(), packed);
+  mf_status pst = mf::pack_instances(ctx, sub.data(), (int32_t)sub.size(), o.batch_mode == 0,
+                                      packed);
   if (pst != MF_OK) return pst;
   mf::BatchResident *resident = nullptr;
   pst = mf::batch_upload(ctx, &packed.view, packed.src.data(), packed.snk.data(),

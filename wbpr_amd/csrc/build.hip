@@ -93,7 +93,8 @@ __global__ void k_in_before(const int *off, const int *in_off, const int *in_lis
   }
 }
 
-// Slot pair of every arc; layout 1 = BCSR ({dst, residual} + rev), 2 = BCSR2 (dst + {residual, rev}).
+// Slot pair of every arc.  A capacity stored as ~c (negative) belongs to an instance solved in the
+// other direction: its reverse slot starts with the residual c.  layout 1 = BCSR ({dst, residual} + rev), 2 = BCSR2 (dst + {residual, rev}).
 __global__ void k_place_slots(const int *off, const int *dst, const int *cap, const int *tail,
                               const int *in_off, const int *in_list, const int *pos_in,
                               const int *in_before, int64_t m, int layout, int2 *dc, int *rev,
@@ -112,19 +113,20 @@ __global__ void k_place_slots(const int *off, const int *dst, const int *cap, co
     const int ov = off[v], ov1 = off[v + 1];
     const int before = u == v ? i - ov : (i >= ov1 ? ov1 - ov : 0);
     const int b = ov + before + pos_in[i] + (u == v ? 1 : 0);
+    const int fwd = max(c, 0), bwd = c < 0 ? ~c : 0;
     if (layout == 1) {
-      dc[a] = make_int2(v, c);
-      dc[b] = make_int2(u, 0);
+      dc[a] = make_int2(v, fwd);
+      dc[b] = make_int2(u, bwd);
       rev[a] = b;
       rev[b] = a;
     } else {
       dst2[a] = v;
       dst2[b] = u;
-      cr[a] = make_int2(c, b);
-      cr[b] = make_int2(0, a);
+      cr[a] = make_int2(fwd, b);
+      cr[b] = make_int2(bwd, a);
     }
-    cap0[a] = c;
-    cap0[b] = 0;
+    cap0[a] = fwd;
+    cap0[b] = bwd;
     fslot[i] = a;
   }
 }

@@ -47,10 +47,13 @@ struct PackedBatch {
   std::vector<int32_t> src, snk, vbase, own;
   mf_csr view{};
 };
-// Concatenates instances: vertex v of instance i becomes vbase[i] + v (batch.cpp).  The staging
+// Concatenates instances: vertex v of instance i becomes vbase[i] + v (batch.cpp).  reverse: the
+// solve returns values only, so instances may be packed in the cheaper direction (capacities of
+// reversed ones as ~c, for upload's device layout).  The staging
 // buffer is the context's: the packed arrays stay valid until the next call on that context that
 // stages data.
-mf_status pack_instances(mf_context *ctx, const mf_csr *inst, int32_t k, PackedBatch &out);
+mf_status pack_instances(mf_context *ctx, const mf_csr *inst, int32_t k, bool reverse,
+                         PackedBatch &out);
 // Pinned host memory of at least `bytes`, owned by the context and reused by later calls (grown
 // when needed); nullptr if it cannot be allocated.
 void *context_staging(mf_context *ctx, size_t bytes);

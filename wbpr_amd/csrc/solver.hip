@@ -2597,7 +2597,7 @@ static mf_status upload(mf_context *ctx, const mf_csr *c, const int32_t *src, co
   for (int32_t i = 0; i < k; ++i) {
     int64_t sc = 0;
     for (int32_t a = c->offsets[src[i]]; a < c->offsets[src[i] + 1]; ++a)
-      if (c->dst[a] != src[i]) sc += cap[a];
+      if (c->dst[a] != src[i] && cap[a] > 0) sc += cap[a];  // (< 0: reversed, checked when packed)
     if (sc > INT32_MAX) return MF_ERR_OVERFLOW;  // every excess must fit int32
   }
   hipStream_t st = ctx->stream;
