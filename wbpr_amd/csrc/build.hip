@@ -125,9 +125,11 @@ __global__ void k_place_slots(const int *off, const int *dst, const int *cap, co
       cr[a] = make_int2(fwd, b);
       cr[b] = make_int2(bwd, a);
     }
-    cap0[a] = fwd;
-    cap0[b] = bwd;
-    fslot[i] = a;
+    if (cap0) {
+      cap0[a] = fwd;
+      cap0[b] = bwd;
+    }
+    if (fslot) fslot[i] = a;
   }
 }
 
@@ -150,13 +152,13 @@ int grid_for(int64_t work) {
 }
 
 template <class T>
-hipError_t dalloc(T **p, int64_t count) {
-  return hipMalloc((void **)p, sizeof(T) * (size_t)std::max<int64_t>(count, 1));
+hipError_t dalloc(DevPool &pool, T **p, int64_t count) {
+  return pool.alloc((void **)p, sizeof(T) * (size_t)std::max<int64_t>(count, 1));
 }
 
 }  // namespace
 
-mf_status build_layout_device(hipStream_t st, int32_t n, int64_t m, const int *off,
+mf_status build_layout_device(hipStream_t st, DevPool &pool, int32_t n, int64_t m, const int *off,
                               const int *dst, const int *cap, mf_layout layout,
                               const DeviceLayout &out, int *in_off_out) {
   int *tail = nullptr, *iota = nullptr, *heads = nullptr, *in_list = nullptr, *pos_in = nullptr;
@@ -166,13 +168,13 @@ mf_status build_layout_device(hipStream_t st, int32_t n, int64_t m, const int *o
   auto cleanup = [&]() {
     void *ptrs[] = {tail, iota, heads, in_list, pos_in, in_off, in_before, tmp};
     for (void *p : ptrs)
-      if (p) (void)hipFree(p);
+      if (p) pool.release(p);
   };
   do {
-    if (dalloc(&tail, m) != hipSuccess || dalloc(&iota, m) != hipSuccess ||
-        dalloc(&heads, m) != hipSuccess || dalloc(&in_list, m) != hipSuccess ||
-        dalloc(&pos_in, m) != hipSuccess || dalloc(&in_off, (int64_t)n + 1) != hipSuccess ||
-        dalloc(&in_before, (int64_t)n) != hipSuccess) {
+    if (dalloc(pool, &tail, m) != hipSuccess || dalloc(pool, &iota, m) != hipSuccess ||
+        dalloc(pool, &heads, m) != hipSuccess || dalloc(pool, &in_list, m) != hipSuccess ||
+        dalloc(pool, &pos_in, m) != hipSuccess || dalloc(pool, &in_off, (int64_t)n + 1) != hipSuccess ||
+        dalloc(pool, &in_before, (int64_t)n) != hipSuccess) {
       result = MF_ERR_OUT_OF_MEMORY;
       break;
     }
@@ -188,7 +190,7 @@ mf_status build_layout_device(hipStream_t st, int32_t n, int64_t m, const int *o
     if (rocprim::radix_sort_pairs(nullptr, tmp_bytes, keys_in, keys_out, iota, in_list,
                                   (size_t)m, 0, bits, st) != hipSuccess)
       break;
-    if (hipMalloc(&tmp, std::max<size_t>(tmp_bytes, 1)) != hipSuccess) {
+    if (pool.alloc(&tmp, std::max<size_t>(tmp_bytes, 1)) != hipSuccess) {
       result = MF_ERR_OUT_OF_MEMORY;
       break;
     }

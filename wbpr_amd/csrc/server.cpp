@@ -403,6 +403,8 @@ mf_status mf_server_create(mf_context *ctx, int64_t hbm_budget_bytes, int32_t ma
       serve_arena_destroy(srv->arena);
       return s;
     }
+    // what the worker contexts keep between requests: an eighth of their half of the budget
+    context_pool_limit(c, (size_t)(srv->alone_budget / (8 * max_inflight_launches)));
     srv->ctxs.push_back(c);
     srv->ctx_busy.push_back(false);
   }

@@ -34,6 +34,7 @@
 #include <vector>
 
 #include "build.h"
+#include "dev_pool.h"
 #include "kernels.h"
 #include "mf_internal.h"
 #include "solver.h"
@@ -2266,14 +2267,6 @@ constexpr int kBfsBlocksPerCU = 2;
 constexpr int kCoopBlocks = 64;
 constexpr long long kCoopSlots = 1 << 17;
 
-template <class T>
-static mf_status dmalloc(T **p, size_t count) {
-  *p = nullptr;
-  if (count == 0) count = 1;
-  HIP_TRY(hipMalloc((void **)p, sizeof(T) * count));
-  return MF_OK;
-}
-
 constexpr int kHubClass = 4;  // first degree class above 1,024 slots (class_config)
 
 static_assert(kClasses == kNumClasses, "host and device class counts differ");
@@ -2372,12 +2365,21 @@ struct mf_context {
   size_t staging_bytes = 0;
   bool cooperative = false;  // the device runs cooperative launches
   int lds_limit = 0;         // LDS of one workgroup, bytes
+  mf::DevPool pool;          // device memory of its calls and graphs
 };
 
 namespace mf {
 
+template <class T>
+static mf_status dmalloc(mf_context *ctx, T **p, size_t count) {
+  *p = nullptr;
+  HIP_TRY(ctx->pool.alloc((void **)p, sizeof(T) * std::max<size_t>(count, 1)));
+  return MF_OK;
+}
+
 // Device-resident residual graph of k packed instances.
 struct DevGraph {
+  mf_context *owner = nullptr;  // whose pool the arrays came from (compared, never followed)
   mf_layout layout = MF_LAYOUT_BCSR;
   int32_t n = 0;  // vertices of all instances
   int64_t m = 0, S = 0;
@@ -2454,7 +2456,8 @@ enum {
 // counter c of triple-buffer slot q of the frontier (CTL_FCNT) or worklist (CTL_CCNT) set
 constexpr int ctl_cnt(int set, int q, int c) { return set + (q * kNumClasses + c) * kCtlStride; }
 
-static void free_dev(DevGraph *g) {
+static void free_dev(mf_context *ctx, DevGraph *g) {
+  (void)hipStreamSynchronize(ctx->stream);  // (after an error)
   for (auto &cg : g->cycle_graphs)
     for (hipGraphExec_t x : cg.exec)
       if (x) (void)hipGraphExecDestroy(x);
@@ -2465,7 +2468,10 @@ static void free_dev(DevGraph *g) {
                   g->work, g->work_cls, g->cycle_base, g->cls_tab, g->giant, g->dirty,
                   g->bu_rem};
   for (void *p : ptrs)
-    if (p) (void)hipFree(p);
+    if (p) {
+      if (ctx == g->owner) ctx->pool.release(p);
+      else (void)hipFree(p);
+    }
 }
 
 // Sums the spread statistics copies (see block_flush).
@@ -2482,13 +2488,13 @@ static hipError_t read_stats(const unsigned long long *dev, unsigned long long o
 
 // Degree classes of every vertex (VC buckets) and the class-grouped order of the vertices of
 // nonzero degree that bottom-up BFS levels walk.  degree counts residual slots.
-static mf_status set_vertex_classes(DevGraph &G, const std::vector<int64_t> &degree,
-                                    hipStream_t st) {
+static mf_status set_vertex_classes(mf_context *ctx, DevGraph &G,
+                                    const std::vector<int64_t> &degree, hipStream_t st) {
   const int n = G.n;
   mf_status rc;
   // (arrays already placed by the caller, as in the static-scratch upload, are used as they are)
-  if ((!G.vcls && (rc = dmalloc(&G.vcls, (size_t)n))) ||
-      (!G.vorder && (rc = dmalloc(&G.vorder, (size_t)std::max(n, 1)))))
+  if ((!G.vcls && (rc = dmalloc(ctx, &G.vcls, (size_t)n))) ||
+      (!G.vorder && (rc = dmalloc(ctx, &G.vorder, (size_t)std::max(n, 1)))))
     return rc;
   const ClassConfig vc = class_config(MF_ALGO_VC, 0);
   std::vector<unsigned char> cls((size_t)n);
@@ -2533,7 +2539,7 @@ static mf_status set_vertex_classes(DevGraph &G, const std::vector<int64_t> &deg
   // giant-list state, one entry per possible list position: no minimum, no parts, nothing
   // reserved (each giant's last part restores this)
   const size_t giants = (size_t)std::max<int64_t>(G.vc_pop[kNumClasses - 1], 1);
-  if (!G.giant && (rc = dmalloc(&G.giant, giants * kGiantWords))) return rc;
+  if (!G.giant && (rc = dmalloc(ctx, &G.giant, giants * kGiantWords))) return rc;
   std::vector<unsigned long long> gs0(giants * kGiantWords, 0ull);
   for (size_t q = 0; q < giants; ++q) gs0[q * kGiantWords] = ~0ull;
   HIP_TRY(hipMemcpy(G.giant, gs0.data(), sizeof(unsigned long long) * gs0.size(),
@@ -2571,11 +2577,17 @@ static mf_status set_vertex_classes(DevGraph &G, const std::vector<int64_t> &deg
   return MF_OK;
 }
 
-// Uploads a (packed) graph: c is the union CSR, src/snk the k terminal pairs.
-// keep_host: keep host copies of the CSR for flow read-back (single solves); batched uploads,
-// whose flows are never read, skip them.
+// What an upload keeps beside the residual layout: a single graph everything; a batch no host copy of
+// the CSR (its flows are never read), and no degree-class tables and worklists unless a kernel
+// that uses them will solve it; a batch solved once no capacities to restart from either.  (4,096
+// matchings of 256 to 65,536 vertices a side: the tables were 300 of a call's 720 ms, on the host.)
+enum class Keep { kAll, kBatchTables, kBatch, kBatchOnce };
+
 static mf_status upload(mf_context *ctx, const mf_csr *c, const int32_t *src, const int32_t *snk,
-                        int32_t k, mf_layout layout, DevGraph &G, bool keep_host = true) {
+                        int32_t k, mf_layout layout, DevGraph &G, Keep keep = Keep::kAll) {
+  const bool keep_host = keep == Keep::kAll;
+  const bool tables = keep == Keep::kAll || keep == Keep::kBatchTables;
+  G.owner = ctx;
   G.layout = layout;
   G.n = c->n;
   G.m = c->m;
@@ -2602,17 +2614,18 @@ static mf_status upload(mf_context *ctx, const mf_csr *c, const int32_t *src, co
   }
   hipStream_t st = ctx->stream;
   if (2 * c->m > INT32_MAX) return MF_ERR_OVERFLOW;
-  std::vector<int64_t> degree((size_t)c->n, 0);
+  std::vector<int64_t> degree(tables ? (size_t)c->n : 0, 0);
   mf_status rc;
   // the CSR goes to the device as it is; the residual layout is built there (build.hip)
   int *d_off = nullptr, *d_dst = nullptr, *d_cap = nullptr;
   auto free_raw = [&]() {
-    if (d_off && d_off != G.off) (void)hipFree(d_off);
-    if (d_dst) (void)hipFree(d_dst);
-    if (d_cap) (void)hipFree(d_cap);
+    (void)hipStreamSynchronize(st);
+    if (d_off && d_off != G.off) ctx->pool.release(d_off);
+    if (d_dst) ctx->pool.release(d_dst);
+    if (d_cap) ctx->pool.release(d_cap);
   };
-  if ((rc = dmalloc(&d_off, (size_t)c->n + 1)) || (rc = dmalloc(&d_dst, (size_t)c->m)) ||
-      (rc = dmalloc(&d_cap, (size_t)c->m))) {
+  if ((rc = dmalloc(ctx, &d_off, (size_t)c->n + 1)) || (rc = dmalloc(ctx, &d_dst, (size_t)c->m)) ||
+      (rc = dmalloc(ctx, &d_cap, (size_t)c->m))) {
     free_raw();
     return rc;
   }
@@ -2628,9 +2641,9 @@ static mf_status upload(mf_context *ctx, const mf_csr *c, const int32_t *src, co
   if (layout == MF_LAYOUT_RCSR) {
     G.S = c->m;
     G.off = d_off;  // RCSR keeps the arc offsets
-    if ((rc = dmalloc(&G.fdc, (size_t)c->m)) || (rc = dmalloc(&G.bcf, (size_t)c->m)) ||
-        (rc = dmalloc(&G.roff, (size_t)c->n + 1)) || (rc = dmalloc(&G.rdi, (size_t)c->m)) ||
-        (rc = dmalloc(&G.cap0, (size_t)c->m))) {
+    if ((rc = dmalloc(ctx, &G.fdc, (size_t)c->m)) || (rc = dmalloc(ctx, &G.bcf, (size_t)c->m)) ||
+        (rc = dmalloc(ctx, &G.roff, (size_t)c->n + 1)) || (rc = dmalloc(ctx, &G.rdi, (size_t)c->m)) ||
+        (rc = dmalloc(ctx, &G.cap0, (size_t)c->m))) {
       free_raw();
       return rc;
     }
@@ -2640,8 +2653,9 @@ static mf_status upload(mf_context *ctx, const mf_csr *c, const int32_t *src, co
     out.cap0 = G.cap0;
   } else {
     G.S = 2 * c->m;
-    if ((rc = dmalloc(&G.off, (size_t)c->n + 1)) || (rc = dmalloc(&G.cap0, (size_t)G.S)) ||
-        (rc = dmalloc(&G.fslot, (size_t)c->m))) {
+    if ((rc = dmalloc(ctx, &G.off, (size_t)c->n + 1)) ||
+        (keep != Keep::kBatchOnce && (rc = dmalloc(ctx, &G.cap0, (size_t)G.S))) ||
+        (keep_host && (rc = dmalloc(ctx, &G.fslot, (size_t)c->m)))) {
       free_raw();
       return rc;
     }
@@ -2649,13 +2663,13 @@ static mf_status upload(mf_context *ctx, const mf_csr *c, const int32_t *src, co
     out.cap0 = G.cap0;
     out.fslot = G.fslot;
     if (layout == MF_LAYOUT_BCSR) {
-      rc = dmalloc(&G.dc, (size_t)G.S);
-      if (rc == MF_OK) rc = dmalloc(&G.rev, (size_t)G.S);
+      rc = dmalloc(ctx, &G.dc, (size_t)G.S);
+      if (rc == MF_OK) rc = dmalloc(ctx, &G.rev, (size_t)G.S);
       out.dc = G.dc;
       out.rev = G.rev;
     } else {
-      rc = dmalloc(&G.dst, (size_t)G.S);
-      if (rc == MF_OK) rc = dmalloc(&G.cr, (size_t)G.S);
+      rc = dmalloc(ctx, &G.dst, (size_t)G.S);
+      if (rc == MF_OK) rc = dmalloc(ctx, &G.cr, (size_t)G.S);
       out.dst2 = G.dst;
       out.cr = G.cr;
     }
@@ -2664,34 +2678,42 @@ static mf_status upload(mf_context *ctx, const mf_csr *c, const int32_t *src, co
       return rc;
     }
   }
-  std::vector<int> in_off((size_t)c->n + 1);
-  rc = build_layout_device(st, c->n, c->m, d_off, d_dst, d_cap, layout, out, in_off.data());
+  std::vector<int> in_off(tables ? (size_t)c->n + 1 : 0);
+  rc = build_layout_device(st, ctx->pool, c->n, c->m, d_off, d_dst, d_cap, layout, out,
+                           tables ? in_off.data() : nullptr);
   free_raw();
   if (rc != MF_OK) return rc;
-  parallel_for(c->n, [&](int64_t b, int64_t e) {
-    for (int64_t v = b; v < e; ++v)
-      degree[(size_t)v] = (int64_t)(c->offsets[v + 1] - c->offsets[v]) +
-                          (in_off[(size_t)v + 1] - in_off[(size_t)v]);
-  });
-  G.degree.resize((size_t)c->n);
-  parallel_for(c->n, [&](int64_t b, int64_t e) {
-    for (int64_t v = b; v < e; ++v) G.degree[(size_t)v] = (int32_t)degree[(size_t)v];
-  });
-  if ((rc = dmalloc(&G.h, (size_t)c->n)) || (rc = dmalloc(&G.e, (size_t)c->n)) ||
-      (rc = dmalloc(&G.stamp, (size_t)c->n)) || (rc = dmalloc(&G.cycle_base, 1)) ||
-      (rc = dmalloc(&G.cls_tab, (size_t)4 * kNumClasses)) ||
-      (rc = dmalloc(&G.lists, (size_t)4 * c->n)) || (rc = dmalloc(&G.ctl, (size_t)CTL_SIZE)) ||
-      (rc = dmalloc(&G.stats, (size_t)kStatSlot * kStatSpread)) || (rc = dmalloc(&G.src, (size_t)k)) ||
-      (rc = dmalloc(&G.snk, (size_t)k)) || (rc = dmalloc(&G.values, (size_t)k)))
+  if (tables) {
+    parallel_for(c->n, [&](int64_t b, int64_t e) {
+      for (int64_t v = b; v < e; ++v)
+        degree[(size_t)v] = (int64_t)(c->offsets[v + 1] - c->offsets[v]) +
+                            (in_off[(size_t)v + 1] - in_off[(size_t)v]);
+    });
+    G.degree.resize((size_t)c->n);
+    parallel_for(c->n, [&](int64_t b, int64_t e) {
+      for (int64_t v = b; v < e; ++v) G.degree[(size_t)v] = (int32_t)degree[(size_t)v];
+    });
+  }
+  if ((rc = dmalloc(ctx, &G.h, (size_t)c->n)) || (rc = dmalloc(ctx, &G.e, (size_t)c->n)) ||
+      (rc = dmalloc(ctx, &G.stamp, (size_t)c->n)) || (rc = dmalloc(ctx, &G.cycle_base, 1)) ||
+      (rc = dmalloc(ctx, &G.cls_tab, (size_t)4 * kNumClasses)) ||
+      (tables && (rc = dmalloc(ctx, &G.lists, (size_t)4 * c->n))) ||
+      (rc = dmalloc(ctx, &G.ctl, (size_t)CTL_SIZE)) ||
+      (rc = dmalloc(ctx, &G.stats, (size_t)kStatSlot * kStatSpread)) ||
+      (rc = dmalloc(ctx, &G.src, (size_t)k)) || (rc = dmalloc(ctx, &G.snk, (size_t)k)) ||
+      (rc = dmalloc(ctx, &G.values, (size_t)k)))
     return rc;
-  if ((rc = set_vertex_classes(G, degree, st)) != MF_OK) return rc;
-  G.max_src_deg = 0;
-  for (int32_t i = 0; i < k; ++i) G.max_src_deg = std::max(G.max_src_deg, degree[(size_t)src[i]]);
+  if (tables) {
+    if ((rc = set_vertex_classes(ctx, G, degree, st)) != MF_OK) return rc;
+    G.max_src_deg = 0;
+    for (int32_t i = 0; i < k; ++i)
+      G.max_src_deg = std::max(G.max_src_deg, degree[(size_t)src[i]]);
+  }
   HIP_TRY(hipMemcpyAsync(G.src, src, sizeof(int) * k, hipMemcpyHostToDevice, st));
   HIP_TRY(hipMemcpyAsync(G.snk, snk, sizeof(int) * k, hipMemcpyHostToDevice, st));
   HIP_TRY(hipMemsetAsync(G.ctl, 0, sizeof(int) * CTL_SIZE, st));
   if (keep_host && G.nonzero >= kBottomUpMinVertices) {  // bottom-up levels' unreached lists
-    if ((rc = dmalloc(&G.bu_rem, (size_t)2 * G.nonzero + 2 * kNumClasses))) return rc;
+    if ((rc = dmalloc(ctx, &G.bu_rem, (size_t)2 * G.nonzero + 2 * kNumClasses))) return rc;
     int tab[2 * kNumClasses];
     for (int c = 0; c < kNumClasses; ++c) {
       tab[c] = G.vo.cls_off[c];
@@ -2700,7 +2722,7 @@ static mf_status upload(mf_context *ctx, const mf_csr *c, const int32_t *src, co
     HIP_TRY(hipMemcpyAsync(G.bu_rem + 2 * G.nonzero, tab, sizeof(tab), hipMemcpyHostToDevice, st));
   }
   if (keep_host && layout != MF_LAYOUT_RCSR && G.S >= kDirtyMinSlots) {  // single graphs only
-    if ((rc = dmalloc(&G.dirty, (size_t)(G.S + 7) / 8))) return rc;
+    if ((rc = dmalloc(ctx, &G.dirty, (size_t)(G.S + 7) / 8))) return rc;
     HIP_TRY(hipMemsetAsync(G.dirty, 0, (size_t)(G.S + 7) / 8, st));
   }
   HIP_TRY(hipStreamSynchronize(st));
@@ -2921,13 +2943,13 @@ static mf_status run_solve(mf_context *ctx, DevGraph &G, const L &lay, mf_algo a
   if (o.record_workload) {  // per-wave busy cycles, summed over this solve's cycle launches
     const int64_t waves = (int64_t)grid * (kBlock / 64);
     if (G.work_waves != waves) {
-      if (G.work) (void)hipFree(G.work);
-      if (G.work_cls) (void)hipFree(G.work_cls);
+      if (G.work) ctx->pool.release(G.work);
+      if (G.work_cls) ctx->pool.release(G.work_cls);
       G.work = nullptr;
       G.work_cls = nullptr;
       G.work_waves = 0;
       mf_status rc;
-      if ((rc = dmalloc(&G.work, (size_t)waves)) || (rc = dmalloc(&G.work_cls, (size_t)waves)))
+      if ((rc = dmalloc(ctx, &G.work, (size_t)waves)) || (rc = dmalloc(ctx, &G.work_cls, (size_t)waves)))
         return rc;
       G.work_waves = waves;
     }
@@ -3412,15 +3434,16 @@ static mf_status run_batch_wg(mf_context *ctx, DevGraph &G, const int32_t *vbase
   int *d_vbase = nullptr, *d_nver = nullptr, *d_pop = nullptr, *d_bpop = nullptr,
       *d_order = nullptr, *d_next = nullptr, *d_status = nullptr;
   auto cleanup = [&]() {
+    (void)hipStreamSynchronize(st);
     for (void *p : {(void *)d_vbase, (void *)d_nver, (void *)d_pop, (void *)d_bpop,
                     (void *)d_order, (void *)d_next, (void *)d_status})
-      if (p) (void)hipFree(p);
+      if (p) ctx->pool.release(p);
   };
   mf_status rc;
-  if ((rc = dmalloc(&d_vbase, (size_t)k)) || (rc = dmalloc(&d_nver, (size_t)k)) ||
-      (rc = dmalloc(&d_pop, (size_t)k * kNumClasses)) ||
-      (rc = dmalloc(&d_bpop, (size_t)k * kNumClasses)) || (rc = dmalloc(&d_order, (size_t)k)) ||
-      (rc = dmalloc(&d_next, (size_t)3)) || (rc = dmalloc(&d_status, (size_t)k))) {
+  if ((rc = dmalloc(ctx, &d_vbase, (size_t)k)) || (rc = dmalloc(ctx, &d_nver, (size_t)k)) ||
+      (rc = dmalloc(ctx, &d_pop, (size_t)k * kNumClasses)) ||
+      (rc = dmalloc(ctx, &d_bpop, (size_t)k * kNumClasses)) || (rc = dmalloc(ctx, &d_order, (size_t)k)) ||
+      (rc = dmalloc(ctx, &d_next, (size_t)3)) || (rc = dmalloc(ctx, &d_status, (size_t)k))) {
     cleanup();
     return rc;
   }
@@ -3547,6 +3570,13 @@ static mf_status run_batch_wg(mf_context *ctx, DevGraph &G, const int32_t *vbase
   return result;
 }
 
+// Whether an instance is too large for the LDS kernels (k_batch_wg needs the degree-class tables).
+static bool batch_has_huge(const mf_context *ctx, const int32_t *vbase, int32_t k) {
+  for (int32_t i = 0; i < k; ++i)
+    if (!wg_batch_takes(vbase[i + 1] - vbase[i], ctx->lds_limit)) return true;
+  return false;
+}
+
 mf_status batch_solve_packed(mf_context *ctx, const mf_csr *packed, const int32_t *src,
                              const int32_t *snk, const int32_t *vbase, int32_t k, mf_algo algo,
                              mf_layout layout, const mf_options &o, int64_t *values,
@@ -3557,7 +3587,8 @@ mf_status batch_solve_packed(mf_context *ctx, const mf_csr *packed, const int32_
   DevGraph G;
   const bool per_group = o.batch_mode == 0;
   const double t0 = now_ms();
-  st = upload(ctx, packed, src, snk, k, per_group ? MF_LAYOUT_BCSR : layout, G, false);
+  st = upload(ctx, packed, src, snk, k, per_group ? MF_LAYOUT_BCSR : layout, G,
+              !per_group || batch_has_huge(ctx, vbase, k) ? Keep::kBatchTables : Keep::kBatchOnce);
   const double t1 = now_ms();
   if (st == MF_OK)
     st = per_group ? run_batch_wg(ctx, G, vbase, algo, o, res) : solve_graph(ctx, G, algo, o, res);
@@ -3568,11 +3599,12 @@ mf_status batch_solve_packed(mf_context *ctx, const mf_csr *packed, const int32_
       st = MF_ERR_DEVICE;
     for (int32_t i = 0; i < k; ++i) values[i] = v[(size_t)i];
   }
-  free_dev(&G);
+  free_dev(ctx, &G);
   return st;
 }
 
 struct BatchResident {
+  mf_context *ctx = nullptr;
   DevGraph G;
   std::vector<int32_t> vbase;
   int32_t k = 0;
@@ -3586,10 +3618,13 @@ mf_status batch_upload(mf_context *ctx, const mf_csr *packed, const int32_t *src
   *out = nullptr;
   HIP_TRY(hipSetDevice(ctx->device));
   BatchResident *r = new BatchResident;
+  r->ctx = ctx;
   r->vbase.assign(vbase, vbase + (size_t)k + 1);
   r->k = k;
   r->batch_mode = o.batch_mode;
-  const mf_status st = upload(ctx, packed, src, snk, k, MF_LAYOUT_BCSR, r->G, false);
+  const mf_status st =
+      upload(ctx, packed, src, snk, k, MF_LAYOUT_BCSR, r->G,
+             o.batch_mode != 0 || batch_has_huge(ctx, vbase, k) ? Keep::kBatchTables : Keep::kBatch);
   if (st != MF_OK) {
     batch_release(r);
     return st;
@@ -3621,7 +3656,7 @@ mf_status batch_solve_resident(mf_context *ctx, BatchResident *r, const mf_optio
 
 void batch_release(BatchResident *r) {
   if (!r) return;
-  free_dev(&r->G);
+  free_dev(r->ctx, &r->G);
   delete r;
 }
 
@@ -3690,12 +3725,17 @@ mf_status serve_arena_create(mf_context *ctx, int64_t nv, int64_t ns, int32_t qc
     serve_arena_destroy(a);
     return r;
   };
-  if ((rc = dmalloc(&a->off, (size_t)nv + 1)) || (rc = dmalloc(&a->rev, (size_t)ns)) ||
-      (rc = dmalloc(&a->h, (size_t)nv)) || (rc = dmalloc(&a->e, (size_t)nv)) ||
-      (rc = dmalloc(&a->stamp, (size_t)nv)) || (rc = dmalloc(&a->lists, (size_t)4 * nv)) ||
-      (rc = dmalloc(&a->dc, (size_t)ns)) || (rc = dmalloc(&a->vcls, (size_t)nv)) ||
-      (rc = dmalloc(&a->words, (size_t)64)) ||
-      (rc = dmalloc(&a->stats, (size_t)kStatSlot * kStatSpread)))
+  // (not from the context's pool: the server's calls come from any thread)
+  auto raw = [](auto **p, size_t count) -> mf_status {
+    HIP_TRY(hipMalloc((void **)p, sizeof(**p) * count));
+    return MF_OK;
+  };
+  if ((rc = raw(&a->off, (size_t)nv + 1)) || (rc = raw(&a->rev, (size_t)ns)) ||
+      (rc = raw(&a->h, (size_t)nv)) || (rc = raw(&a->e, (size_t)nv)) ||
+      (rc = raw(&a->stamp, (size_t)nv)) || (rc = raw(&a->lists, (size_t)4 * nv)) ||
+      (rc = raw(&a->dc, (size_t)ns)) || (rc = raw(&a->vcls, (size_t)nv)) ||
+      (rc = raw(&a->words, (size_t)64)) ||
+      (rc = raw(&a->stats, (size_t)kStatSlot * kStatSpread)))
     return fail(rc);
   if (hipHostMalloc((void **)&a->entries, sizeof(int) * kServeEntryInts * (size_t)qcap,
                     hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess ||
@@ -3817,6 +3857,8 @@ bool serve_running(ServeArena *a) {
 int64_t serve_launches(const ServeArena *a) { return a->launches; }
 
 int context_device(const mf_context *ctx) { return ctx->device; }
+
+void context_pool_limit(mf_context *ctx, size_t bytes) { ctx->pool.limit = bytes; }
 
 void *context_staging(mf_context *ctx, size_t bytes) {
   if (ctx->staging_bytes >= bytes) return ctx->staging;
@@ -4000,7 +4042,7 @@ static mf_status upload_static(mf_context *ctx, const mf_csr *c, DevGraph &G) {
   // control words start at zero (the previous call on this device left its own): a fill kernel
   k_fill_int<<<1, 256, 0, st>>>(G.ctl, 0, CTL_SIZE);
   HIP_TRY(hipGetLastError());
-  if ((rc = set_vertex_classes(G, degree, st)) != MF_OK) return rc;
+  if ((rc = set_vertex_classes(ctx, G, degree, st)) != MF_OK) return rc;
   G.max_src_deg = degree[(size_t)c->s];
   HIP_TRY(hipStreamSynchronize(st));
   G.fresh = true;  // the residuals were written as the capacities
@@ -4056,6 +4098,7 @@ mf_status mf_context_create(int device, mf_context **out) {
 mf_status mf_context_destroy(mf_context *ctx) {
   if (!ctx) return MF_ERR_INVALID_ARGUMENT;
   (void)hipSetDevice(ctx->device);
+  ctx->pool.trim();
   for (hipEvent_t e : ctx->prof_ev) (void)hipEventDestroy(e);
   for (hipEvent_t e : ctx->ev_solve)
     if (e) (void)hipEventDestroy(e);
@@ -4090,7 +4133,7 @@ mf_status mf_graph_upload(mf_context *ctx, const mf_csr *g, mf_layout layout, mf
   const int32_t s = g->s, t = g->t;
   st = upload(ctx, g, &s, &t, 1, layout, mg->g);
   if (st != MF_OK) {
-    free_dev(&mg->g);
+    free_dev(ctx, &mg->g);
     delete mg;
     return st;
   }
@@ -4241,7 +4284,7 @@ mf_status mf_graph_read_state(mf_context *ctx, mf_graph *mg, int32_t *height, in
 mf_status mf_graph_destroy(mf_context *ctx, mf_graph *mg) {
   if (!ctx || !mg) return MF_ERR_INVALID_ARGUMENT;
   (void)hipSetDevice(ctx->device);
-  free_dev(&mg->g);
+  free_dev(ctx, &mg->g);
   delete mg;
   return MF_OK;
 }
@@ -4324,6 +4367,7 @@ mf_status mf_rcsr_push_relabel(mf_context *ctx, int algo_type, int V, int E, int
   HIP_TRY(hipSetDevice(ctx->device));
   DevGraph G;
   hipStream_t s = ctx->stream;
+  G.owner = ctx;
   G.layout = MF_LAYOUT_RCSR;
   G.n = V;
   G.m = E;
@@ -4338,28 +4382,28 @@ mf_status mf_rcsr_push_relabel(mf_context *ctx, int algo_type, int V, int E, int
   for (int32_t i = cpu_offsets[source]; i < cpu_offsets[source + 1]; ++i)
     if (cpu_destinations[i] != source) sc += cpu_capacities[i];
   auto fail = [&](mf_status code) {
-    free_dev(&G);
+    free_dev(ctx, &G);
     return code;
   };
   if (sc > INT32_MAX) return fail(MF_ERR_OVERFLOW);
   std::vector<int2> fdc((size_t)E), rdi((size_t)E);
   for (int i = 0; i < E; ++i) fdc[(size_t)i] = make_int2(cpu_destinations[i], cpu_capacities[i]);
   for (int q = 0; q < E; ++q) rdi[(size_t)q] = make_int2(cpu_rdestinations[q], cpu_flow_idx[q]);
-  if ((st = dmalloc(&G.off, (size_t)V + 1)) || (st = dmalloc(&G.fdc, (size_t)E)) ||
-      (st = dmalloc(&G.bcf, (size_t)E)) || (st = dmalloc(&G.roff, (size_t)V + 1)) ||
-      (st = dmalloc(&G.rdi, (size_t)E)) || (st = dmalloc(&G.cap0, (size_t)E)) ||
-      (st = dmalloc(&G.h, (size_t)V)) || (st = dmalloc(&G.e, (size_t)V)) ||
-      (st = dmalloc(&G.stamp, (size_t)V)) || (st = dmalloc(&G.cycle_base, 1)) ||
-      (st = dmalloc(&G.cls_tab, (size_t)4 * kNumClasses)) ||
-      (st = dmalloc(&G.lists, (size_t)4 * V)) || (st = dmalloc(&G.ctl, (size_t)CTL_SIZE)) ||
-      (st = dmalloc(&G.stats, (size_t)kStatSlot * kStatSpread)) || (st = dmalloc(&G.src, (size_t)1)) ||
-      (st = dmalloc(&G.snk, (size_t)1)) || (st = dmalloc(&G.values, (size_t)1)))
+  if ((st = dmalloc(ctx, &G.off, (size_t)V + 1)) || (st = dmalloc(ctx, &G.fdc, (size_t)E)) ||
+      (st = dmalloc(ctx, &G.bcf, (size_t)E)) || (st = dmalloc(ctx, &G.roff, (size_t)V + 1)) ||
+      (st = dmalloc(ctx, &G.rdi, (size_t)E)) || (st = dmalloc(ctx, &G.cap0, (size_t)E)) ||
+      (st = dmalloc(ctx, &G.h, (size_t)V)) || (st = dmalloc(ctx, &G.e, (size_t)V)) ||
+      (st = dmalloc(ctx, &G.stamp, (size_t)V)) || (st = dmalloc(ctx, &G.cycle_base, 1)) ||
+      (st = dmalloc(ctx, &G.cls_tab, (size_t)4 * kNumClasses)) ||
+      (st = dmalloc(ctx, &G.lists, (size_t)4 * V)) || (st = dmalloc(ctx, &G.ctl, (size_t)CTL_SIZE)) ||
+      (st = dmalloc(ctx, &G.stats, (size_t)kStatSlot * kStatSpread)) || (st = dmalloc(ctx, &G.src, (size_t)1)) ||
+      (st = dmalloc(ctx, &G.snk, (size_t)1)) || (st = dmalloc(ctx, &G.values, (size_t)1)))
     return fail(st);
   std::vector<int64_t> degree((size_t)V);
   for (int32_t v = 0; v < V; ++v)
     degree[(size_t)v] = (int64_t)(cpu_offsets[v + 1] - cpu_offsets[v]) +
                         (cpu_roffsets[v + 1] - cpu_roffsets[v]);
-  if ((st = set_vertex_classes(G, degree, s)) != MF_OK) return fail(st);
+  if ((st = set_vertex_classes(ctx, G, degree, s)) != MF_OK) return fail(st);
   G.max_src_deg = degree[(size_t)source];
   // copies of the per-arc arrays only when there are arcs (their pointers may be NULL then)
   auto put = [&](void *dst, const void *src, size_t bytes) {
