@@ -19,15 +19,11 @@ namespace mf {
 // flow value is that of the reversed network, and the excess that can never arrive -- the preflow
 // beyond the terminal's capacity, which would move about until a global relabel finds it cut off
 // -- is not pushed at all (1,024 matchings of 256 to 65,536 vertices a side: 62 M -> 15 M discharges,
-// 73 -> 17 ms).  Less than one part in kReverseMargin apart nothing is gained, and the direction
-// asked for is kept.
-// A reversed instance's terminals are swapped and its capacities c stored as ~c (negative), which
+// 73 -> 17 ms).  A reversed instance's terminals are swapped and its capacities c stored as ~c (negative), which
 // the device layout turns into residuals on the reverse slots.
 //
 // The arrays go into the context's pinned staging buffer when it can provide one
 // (so the upload is one DMA per array), else into out.own; instances are copied in parallel.
-constexpr int64_t kReverseMargin = 8;
-
 mf_status pack_instances(mf_context *ctx, const mf_csr *inst, int32_t k, bool reverse,
                          PackedBatch &out) {
   int64_t N = 0, M = 0;
@@ -54,7 +50,7 @@ mf_status pack_instances(mf_context *ctx, const mf_csr *inst, int32_t k, bool re
             if (g.dst[a] == g.t) into_t += g.cap ? g.cap[a] : 1;
           for (int32_t a = g.offsets[g.t]; a < g.offsets[g.t + 1]; ++a)
             if (g.dst[a] == g.t) into_t -= g.cap ? g.cap[a] : 1;
-          rev[(size_t)i] = into_t < from_s - from_s / kReverseMargin;
+          rev[(size_t)i] = solves_reversed(from_s, into_t);
         }
       },
       1);

@@ -35,7 +35,7 @@ using namespace mf;
 namespace {
 
 // Requests above either size run alone on the whole grid.
-constexpr int32_t kSoloVertices = 16384;
+constexpr int32_t kSoloVertices = kServeVertices;
 constexpr int64_t kSoloArcs = 262144;
 constexpr int32_t kQueueCap = 4096;    // entries of the serving kernel's queue ring
 constexpr int64_t kSlotsPerVertex = 10;  // arena slot capacity per vertex (S = 2m ~ 10n typical)
@@ -184,6 +184,22 @@ static void finish(mf_server *srv, Request &r, State s) {
   }
 }
 
+// A request solved alone returns a value only: in the direction of less terminal capacity, as
+// pack_instances packs batches (terminals swapped, capacities c stored as ~c).
+static void reverse_if_cheaper(Request &r) {
+  int64_t from_s = 0, into_t = 0;
+  for (int32_t v = 0; v < r.n; ++v)
+    for (int32_t i = r.off[(size_t)v]; i < r.off[(size_t)v + 1]; ++i) {
+      if (r.dst[(size_t)i] == v) continue;
+      if (v == r.s) from_s += r.cap[(size_t)i];
+      if (r.dst[(size_t)i] == r.t) into_t += r.cap[(size_t)i];
+    }
+  // (more than an int32 out of the source is refused as it stands)
+  if (from_s > INT32_MAX || !solves_reversed(from_s, into_t)) return;
+  std::swap(r.s, r.t);
+  for (int32_t &c : r.cap) c = ~c;
+}
+
 static void run_alone(mf_server *srv, Launch *L) {
   Request &r = *L->req;
   const mf_csr c = r.view();
@@ -265,9 +281,6 @@ static void publish_copied(mf_server *srv) {
     if (cs == 0) break;  // copies finish in order on the arena's copy stream
     serve_copy_release(r.copy_done);
     r.copy_done = nullptr;
-    r.inst.a_off.clear();
-    r.inst.a_dc.clear();
-    r.inst.a_rev.clear();
     srv->copying.pop_front();
     if (cs < 0) {
       srv->vranges.release(r.vb, (int64_t)r.inst.n + 1);
@@ -279,7 +292,7 @@ static void publish_copied(mf_server *srv) {
     r.q = srv->next_q++;
     r.state = PUBLISHED;
     r.t_start = now_ms() - srv->t0;
-    serve_publish(srv->arena, r.q, r.inst, r.vb);
+    serve_publish(srv->arena, r.q, r.inst, r.vb, r.sb);
     srv->published.push_back(rp);
   }
 }
@@ -434,6 +447,7 @@ mf_status mf_server_submit(mf_server *srv, const mf_csr *g, int64_t *request_id)
     r->dst.assign(g->dst, g->dst + g->m);
     r->cap.resize((size_t)g->m);
     for (int64_t i = 0; i < g->m; ++i) r->cap[(size_t)i] = g->cap ? g->cap[i] : 1;
+    reverse_if_cheaper(*r);
     r->footprint = mf_footprint_bytes(g->n, g->m);
   }
   std::lock_guard<std::mutex> lk(srv->mu);

@@ -39,6 +39,7 @@
 #include "mf_internal.h"
 #include "solver.h"
 #include "wg_launch.h"
+#include "wg_solve.h"
 
 using namespace mfk;
 
@@ -2038,9 +2039,11 @@ __global__ __launch_bounds__(kBlock) void k_batch_wg(L g, BatchArgs b) {
 // request's residual slots, offsets and vertex classes into its ranges of the server's device
 // arena, then publishes queue entry q: it writes the entry (vertex range, terminals, class
 // populations) and then the published count, both in host memory that the GPU reads uncached.
-// A workgroup claims the next published entry on a device counter, solves the instance exactly
-// like a batched one (batch_instance), and writes the value, status and device times into the
-// entry's report in host memory, the entry number last.  An idle workgroup sleeps between looks
+// A workgroup claims the next published entry on a device counter, solves the instance -- with its
+// vertex state in LDS (wg_solve.h), or like a huge batched one (batch_instance) if a frontier of
+// the first global relabel is wide -- and writes the value, status and device times into the
+// entry's report in host memory, the entry number last.  Instances keep their own vertex and slot
+// ids in the arena: the kernel shifts the arrays' bases to an instance's ranges.  An idle workgroup sleeps between looks
 // at the published count and leaves once it has been idle for idle_ticks, or when the host closes
 // the queue, so the grid drains by itself; the host launches it again when entries are published
 // that no running workgroup will take.
@@ -2053,11 +2056,11 @@ __global__ __launch_bounds__(kBlock) void k_batch_wg(L g, BatchArgs b) {
 // (the last value read is kept in device memory), so the grid does not flood the host link.
 
 struct ServeEntry {
-  int vb, n, s, t;        // vertex range [vb, vb + n) in the arena, source, sink
+  int vb, sb, n, s, t;    // first vertex and slot in the arena, vertices, source, sink (local ids)
   int pop[kNumClasses];   // cycle-class populations of the instance
   int bpop[kNumClasses];  // BFS-class populations
 };
-constexpr int kServeEntryInts = 4 + 2 * kNumClasses;
+constexpr int kServeEntryInts = 5 + 2 * kNumClasses;
 static_assert(sizeof(ServeEntry) == sizeof(int) * kServeEntryInts, "ServeEntry is plain ints");
 
 struct ServeReport {
@@ -2079,6 +2082,9 @@ struct ServeArgs {
   long long *last_claim;       // device memory: wall_clock64 of the last claim or finish
   int *busy;                   // device memory: workgroups solving an instance now
   int qcap;
+  int lds_bytes;               // dynamic LDS of a workgroup
+  float wg_ratio;              // cycle time / relabel time of the LDS solver
+  int wide;                    // frontiers wider than this take batch_instance
   long long idle_ticks;        // ticks without any claim or finish after which idle workgroups
                                // leave (none may be busy)
 };
@@ -2109,6 +2115,8 @@ __global__ __launch_bounds__(kBlock) void k_serve_wg(L g, ServeArgs a) {
   __shared__ int s_q;
   __shared__ int s_tab[2][2 * kNumClasses];
   __shared__ int s_entry[kServeEntryInts];
+  extern __shared__ __align__(16) char lds[];
+  __shared__ WgShared s_wg;
   const int tid = (int)threadIdx.x;
   Stats st{0, 0, 0, 0};
   long long nv = 0, ns = 0;
@@ -2167,17 +2175,37 @@ __global__ __launch_bounds__(kBlock) void k_serve_wg(L g, ServeArgs a) {
     // the request's arena ranges were written by a copy after this kernel may have cached them
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
     __syncthreads();
-    const BatchInst I{s_entry[0], s_entry[1], s_entry[2], s_entry[3], s_entry + 4,
-                      s_entry + 4 + kNumClasses};
-    // host state of the instance's vertices: no excess, never discharged
-    for (int v = I.vb + tid; v < I.vb + I.n; v += kBlock) {
-      a.b.e[v] = 0;
-      a.b.stamp[v] = -1;
-    }
-    __syncthreads();
+    const int vb = s_entry[0], sb = s_entry[1], n = s_entry[2];
+    const LayoutBCSR gi{g.off + vb, g.dc + sb, g.rev + sb, nullptr};
     int status = 0;
-    const long long value =
-        batch_instance(g, a.b, I, &status, s_f, s_c, s_flag, &s_dec, s_tab, st, nv, ns);
+    long long value;
+    {
+      WgSolver<LayoutBCSR, kWgBoth, kBlock> w{gi, s_wg, 0, n, s_entry[3], s_entry[4]};
+      w.st = WgStats{0, 0, 0, 0, 0, 0};
+      w.carve(lds, a.lds_bytes, nullptr, nullptr);
+      const WgOutcome o = w.solve(a.wg_ratio, a.b.max_cycles, a.b.max_rounds, a.wide, 0);
+      value = o.value;
+      status = o.status;
+      st = Stats{w.st.active, w.st.slots, w.st.pushes, w.st.relabels};
+      nv += w.st.bfs_verts;
+      ns += w.st.bfs_slots;
+    }
+    if (status == 3) {
+      BatchArgs b = a.b;
+      b.h += vb;
+      b.e += vb;
+      b.stamp += vb;
+      b.vcls += vb;
+      b.lists += vb;
+      // no excess, never discharged
+      for (int v = tid; v < n; v += kBlock) {
+        b.e[v] = 0;
+        b.stamp[v] = -1;
+      }
+      __syncthreads();
+      const BatchInst I{0, n, s_entry[3], s_entry[4], s_entry + 5, s_entry + 5 + kNumClasses};
+      value = batch_instance(gi, b, I, &status, s_f, s_c, s_flag, &s_dec, s_tab, st, nv, ns);
+    }
     // every write of the instance reaches memory before the host may reuse its ranges
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
     __syncthreads();
@@ -3663,6 +3691,10 @@ void batch_release(BatchResident *r) {
 // ---- serving arena (host side of k_serve_wg) ---------------------------------------------------
 
 constexpr int kServeGroupsPerCU = 1;               // resident serving workgroups per CU
+// LDS of a serving workgroup: the state of the largest instance and its lists.  The rest of a CU's
+// 160 KB stays with the solves that run alone beside it.
+constexpr int kServeLds = 112 << 10;
+static_assert(wg_kind(kServeVertices, kServeLds) == kWgBoth, "every served instance fits");
 constexpr long long kServeIdleTicks = 200000;      // 2 ms at the 100 MHz wall clock
 
 struct ServeArena {
@@ -3765,15 +3797,23 @@ mf_status serve_prepare(const mf_csr *g, ServeInstance &I) {
   const ClassConfig vc = class_config(MF_ALGO_VC, 0);
   I.n = g->n;
   I.S = L.slots;
-  I.s = g->s;
-  I.t = g->t;
+  // a value is all a request returns: with clearly less capacity into t than out of s the reversed
+  // network is laid out (see pack_instances)
+  int64_t from_s = 0, into_t = 0;
+  for (int32_t j = L.off[(size_t)g->s]; j < L.off[(size_t)g->s + 1]; ++j)
+    if (L.dst[(size_t)j] != g->s) from_s += L.cap0[(size_t)j];
+  for (int32_t j = L.off[(size_t)g->t]; j < L.off[(size_t)g->t + 1]; ++j)
+    if (L.dst[(size_t)j] != g->t) into_t += L.cap0[(size_t)L.rev[(size_t)j]];
+  const bool reverse = solves_reversed(from_s, into_t);
+  I.s = reverse ? g->t : g->s;
+  I.t = reverse ? g->s : g->t;
   I.off = std::move(L.off);
-  I.rev = std::move(L.rev);
   I.dc.resize((size_t)(2 * I.S));
   for (int64_t j = 0; j < I.S; ++j) {
     I.dc[(size_t)(2 * j)] = L.dst[(size_t)j];
-    I.dc[(size_t)(2 * j + 1)] = L.cap0[(size_t)j];
+    I.dc[(size_t)(2 * j + 1)] = L.cap0[(size_t)(reverse ? L.rev[(size_t)j] : j)];
   }
+  I.rev = std::move(L.rev);
   I.vcls.resize((size_t)I.n);
   for (int q = 0; q < kNumClasses; ++q) I.pop[q] = I.bpop[q] = 0;
   for (int32_t v = 0; v < I.n; ++v) {
@@ -3789,23 +3829,13 @@ mf_status serve_copy(ServeArena *a, ServeInstance &I, int32_t vb, int64_t sb, vo
   if (vb < 0 || (int64_t)vb + I.n + 1 > a->nv || sb < 0 || sb + I.S > a->ns)
     return MF_ERR_INVALID_ARGUMENT;
   HIP_TRY(hipSetDevice(a->ctx->device));
-  // arena ids: vertices from vb, slots from sb
-  I.a_off.resize((size_t)I.n + 1);
-  for (int32_t v = 0; v <= I.n; ++v) I.a_off[(size_t)v] = (int32_t)(sb + I.off[(size_t)v]);
-  I.a_dc.resize(I.dc.size());
-  I.a_rev.resize(I.rev.size());
-  for (int64_t j = 0; j < I.S; ++j) {
-    I.a_dc[(size_t)(2 * j)] = vb + I.dc[(size_t)(2 * j)];
-    I.a_dc[(size_t)(2 * j + 1)] = I.dc[(size_t)(2 * j + 1)];
-    I.a_rev[(size_t)j] = (int32_t)(sb + I.rev[(size_t)j]);
-  }
   hipStream_t st = a->copy_stream;
-  HIP_TRY(hipMemcpyAsync(a->off + vb, I.a_off.data(), sizeof(int) * ((size_t)I.n + 1),
+  HIP_TRY(hipMemcpyAsync(a->off + vb, I.off.data(), sizeof(int) * ((size_t)I.n + 1),
                          hipMemcpyHostToDevice, st));
   if (I.S) {
-    HIP_TRY(hipMemcpyAsync(a->dc + sb, I.a_dc.data(), sizeof(int2) * (size_t)I.S,
+    HIP_TRY(hipMemcpyAsync(a->dc + sb, I.dc.data(), sizeof(int2) * (size_t)I.S,
                            hipMemcpyHostToDevice, st));
-    HIP_TRY(hipMemcpyAsync(a->rev + sb, I.a_rev.data(), sizeof(int) * (size_t)I.S,
+    HIP_TRY(hipMemcpyAsync(a->rev + sb, I.rev.data(), sizeof(int) * (size_t)I.S,
                            hipMemcpyHostToDevice, st));
   }
   HIP_TRY(hipMemcpyAsync(a->vcls + vb, I.vcls.data(), (size_t)I.n, hipMemcpyHostToDevice, st));
@@ -3829,9 +3859,9 @@ void serve_copy_release(void *done) {
   if (done) (void)hipEventDestroy((hipEvent_t)done);
 }
 
-void serve_publish(ServeArena *a, int64_t q, const ServeInstance &I, int32_t vb) {
+void serve_publish(ServeArena *a, int64_t q, const ServeInstance &I, int32_t vb, int64_t sb) {
   int *en = a->entries + (size_t)(q % a->qcap) * kServeEntryInts;
-  const int vals[kServeEntryInts] = {vb, I.n, vb + I.s, vb + I.t,
+  const int vals[kServeEntryInts] = {vb, (int)sb, I.n, I.s, I.t,
                                      I.pop[0], I.pop[1], I.pop[2], I.pop[3], I.pop[4], I.pop[5],
                                      I.bpop[0], I.bpop[1], I.bpop[2], I.bpop[3], I.bpop[4],
                                      I.bpop[5]};
@@ -3915,9 +3945,14 @@ mf_status serve_launch(ServeArena *a) {
   sa.busy = a->words + 8;
   sa.qcap = a->qcap;
   sa.idle_ticks = kServeIdleTicks;
+  sa.lds_bytes = kServeLds;
+  sa.wg_ratio = kDefaultRelabelRatio;
+  sa.wide = kWgWideBoth;
+  HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(k_serve_wg<LayoutBCSR>),
+                              hipFuncAttributeMaxDynamicSharedMemorySize, kServeLds));
   const int nwg = std::max(1, kServeGroupsPerCU * a->ctx->num_cu);
-  k_serve_wg<LayoutBCSR><<<nwg, kBlock, 0, a->kernel_stream>>>(LayoutBCSR{a->off, a->dc, a->rev},
-                                                               sa);
+  k_serve_wg<LayoutBCSR><<<nwg, kBlock, kServeLds, a->kernel_stream>>>(
+      LayoutBCSR{a->off, a->dc, a->rev, nullptr}, sa);
   HIP_TRY(hipGetLastError());
   a->launched = true;
   a->launches++;
