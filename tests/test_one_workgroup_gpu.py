@@ -33,6 +33,12 @@ def dense_layers(mf, k, layers, seed):
 
 def check(mf, orc, ctx, g):
     value = orc.dinic_maxflow(g)
+    for g2 in (g, mf.Graph.from_arcs(g.n, g.dst, g.tails(), g.cap, g.t, g.s)):
+        # one instance to a CU; in more than there are CUs, with small ones beside
+        assert ctx.batch_solve([g2])[0].tolist() == [value]
+    tiny = chains(mf, 3, 4, seed=1)
+    values = ctx.batch_solve([tiny] * 300 + [g])[0]
+    assert values[300] == value and set(values[:300]) == {orc.dinic_maxflow(tiny)}
     tails = g.tails()
     for layout in (mf.LAYOUT_BCSR, mf.LAYOUT_BCSR2, mf.LAYOUT_RCSR):
         dg = ctx.upload(g, layout)

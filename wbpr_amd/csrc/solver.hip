@@ -1747,6 +1747,12 @@ __global__ __launch_bounds__(kBlock) void k_preflow(L g, int *e, const int *src,
   block_flush(sum, 0, 0, 0, stats, ST_SOURCE_OUT);
 }
 
+// side[v] = 1 where the last global relabel reached v (read_cut of large graphs)
+__global__ void k_cut(const int *h, int n, unsigned char *side) {
+  const int stride = gridDim.x * blockDim.x;
+  for (int v = blockIdx.x * blockDim.x + threadIdx.x; v < n; v += stride) side[v] = h[v] < n;
+}
+
 __global__ void k_set_int(int *p, int v) { *p = v; }
 
 __global__ void k_fill_int(int *p, int v, int count) {
@@ -2295,7 +2301,7 @@ constexpr int kBfsBlocksPerCU = 2;
 constexpr int kCoopBlocks = 64;
 constexpr long long kCoopSlots = 1 << 17;
 
-constexpr int kHubClass = 4;  // first degree class above 1,024 slots (class_config)
+constexpr int kHeavyClass = 3;  // first degree class above 32 slots (class_config)
 
 static_assert(kClasses == kNumClasses, "host and device class counts differ");
 static_assert(kTunedClasses == sizeof(((mf_options *)nullptr)->class_lanes) / sizeof(uint16_t),
@@ -2453,7 +2459,7 @@ struct DevGraph {
   int64_t class_slots[kNumClasses] = {0};  // residual slots of the vertices of each VC class
   int64_t max_src_deg = 0;         // largest residual degree of a source
   int64_t giant_parts = 0;         // parts of all giants (kPartSlots slots each)
-  int64_t inner_hubs = 0;          // single graphs: vertices beside the terminals above 1,024 slots
+  int64_t heavy_slots = 0;         // slots of vertices of more than 32, the terminals aside
   unsigned long long *giant = nullptr;  // per giant-list position: state of the parts
   // host copies for result read-back (single solves; batched uploads keep none)
   std::vector<int32_t> h_off, h_dst, h_cap, h_fslot, h_src, h_snk;
@@ -2560,10 +2566,10 @@ static mf_status set_vertex_classes(mf_context *ctx, DevGraph &G,
     }
     G.giant_parts += pc[4 * kNumClasses];
   }
-  G.inner_hubs = G.vc_pop[kHubClass] + G.vc_pop[kHubClass + 1];
+  for (int q = kHeavyClass; q < kNumClasses; ++q) G.heavy_slots += G.class_slots[q];
   if (G.k == 1)
     for (int32_t v : {G.h_src[0], G.h_snk[0]})
-      if (class_of_degree(vc, degree[(size_t)v]) >= kHubClass) --G.inner_hubs;
+      if (class_of_degree(vc, degree[(size_t)v]) >= kHeavyClass) G.heavy_slots -= degree[(size_t)v];
   // giant-list state, one entry per possible list position: no minimum, no parts, nothing
   // reserved (each giant's last part restores this)
   const size_t giants = (size_t)std::max<int64_t>(G.vc_pop[kNumClasses - 1], 1);
@@ -2782,17 +2788,21 @@ static void restore_residuals(mf_context *ctx, DevGraph &G) {
 // kernels and have no meaning here.  Genrmf 16 x 16 x 16 10.5 -> 2.1 ms, Genrmf 29 x 29 x 47 55 -> 31
 // ms, a 64 x 64 random level graph 9.1 -> 1.7 ms, one of 8 x 8 0.82 -> 0.11 ms.
 //
-// Above kWgNarrowSlots residual slots only graphs without hubs, whose levels scan as much as the
-// grid can take (R-MAT 13, edge factor 8: 0.92 ms there, 1.8 ms here), and only with frontiers that
-// are narrow next to the workgroup, seen in the first global relabel.  With the excesses in LDS too a
-// graph may have kWgWideLevels wide ones -- a matching network has two, and is still solved
-// sooner here: 8,000 + 8,000 vertices 3.8 ms there, 1.6 ms here -- before it counts as wide and
-// deep, work for the whole grid; with the excesses in global memory none (16,000 + 16,000: 3.9 and
-// 3.2 ms, 20,000 + 20,500: 2.3 and 2.8 ms, Genrmf 48 x 48 x 20: 32 and 40 ms).
-constexpr int64_t kWgNarrowSlots = 1 << 15;
+// Above kWgNarrowSlots residual slots only graphs of low degree, whose levels and cycles are small
+// next to their number (R-MAT 12, edge factor 8, 57,000 slots: 0.97 ms on the grid, 0.64 ms here; R-MAT
+// 13, 118,000 slots: 0.90 and 1.7 ms), and only with frontiers that are narrow next to the
+// workgroup, seen in the first global relabel.  With the excesses in LDS too a graph may have
+// kWgWideLevels wide ones -- a matching network has two, and is still solved sooner here: 8,000 +
+// 8,000 vertices 3.8 ms there, 1.6 ms here -- before it counts as wide and deep, work for the whole
+// grid; with the excesses in global memory none (16,000 + 16,000: 3.9 and 3.2 ms, 20,000 + 20,500: 2.3
+// and 2.8 ms, Genrmf 48 x 48 x 20: 32 and 40 ms).
+constexpr int64_t kWgNarrowSlots = 1 << 16;
 constexpr int64_t kWgMaxSlots = 1 << 21;
 constexpr int kWgWideBoth = 2800, kWgWideHeights = 2048;
 constexpr int kWgWideLevels = 2;
+
+// At most an eighth of the slots belong to vertices of more than 32.
+static bool low_degree(const DevGraph &G) { return G.heavy_slots * 8 <= 2 * G.m; }
 
 static bool wg_allowed(const mf_options &o) {
   return !o.verbose && !o.profile_kernels && !o.record_workload && !o.cycle_graphs &&
@@ -2805,8 +2815,9 @@ template <class L>
 static mf_status run_one_workgroup(mf_context *ctx, DevGraph &G, const L &lay, const mf_options &o,
                                    mf_result *res, bool *taken) {
   *taken = false;
-  if (G.k != 1 || !wg_allowed(o) || G.S > kWgMaxSlots ||
-      (G.S > kWgNarrowSlots && G.inner_hubs > 0))
+  const int64_t slots = 2 * G.m;  // (whatever the layout)
+  if (G.k != 1 || !wg_allowed(o) || slots > kWgMaxSlots ||
+      (slots > kWgNarrowSlots && !low_degree(G)))
     return MF_OK;
   const int kind = wg_single_kind(G.n, ctx->lds_limit);
   if (kind < 0) return MF_OK;
@@ -2829,7 +2840,7 @@ static mf_status run_one_workgroup(mf_context *ctx, DevGraph &G, const L &lay, c
   a.max_cycles = o.cycles_per_relabel > 0 ? o.cycles_per_relabel : kMaxAdaptiveCycles;
   a.max_rounds = o.max_rounds > 0 ? o.max_rounds : (int64_t)100000000;
   const bool both = kind == kWgBoth;
-  a.wide = G.S > kWgNarrowSlots ? (both ? kWgWideBoth : kWgWideHeights) : 0;
+  a.wide = slots > kWgNarrowSlots ? (both ? kWgWideBoth : kWgWideHeights) : 0;
   a.wide_levels = both ? kWgWideLevels : 0;
   a.values = G.values;
   static_assert(sizeof(WgReport) <= sizeof(int) * CTL_SIZE, "the report fits the control words");
@@ -4090,6 +4101,11 @@ struct mf_graph {
   mf::DevGraph g;
 };
 
+// From this many vertices mf_graph_read_cut compares on the device and copies a byte per vertex
+// (R-MAT 22: 2.2 -> 0.34 ms, 79,000 vertices 58 -> 41 us); below, a launch costs what the smaller
+// copy saves.
+constexpr int32_t kCutOnDevice = 1 << 16;
+
 using namespace mf;
 
 extern "C" {
@@ -4300,6 +4316,19 @@ mf_status mf_graph_read_cut(mf_context *ctx, mf_graph *mg, uint8_t *sink_side) {
   DevGraph &G = mg->g;
   if (!G.solved) return MF_ERR_INVALID_ARGUMENT;
   HIP_TRY(hipSetDevice(ctx->device));
+  if (G.n >= kCutOnDevice) {
+    unsigned char *side = nullptr;
+    const mf_status rc = dmalloc(ctx, &side, (size_t)G.n);
+    if (rc != MF_OK) return rc;
+    k_cut<<<8 * ctx->num_cu, 256, 0, ctx->stream>>>(G.h, G.n, side);
+    const bool ok = hipGetLastError() == hipSuccess &&
+                    hipMemcpyAsync(sink_side, side, (size_t)G.n, hipMemcpyDeviceToHost,
+                                   ctx->stream) == hipSuccess &&
+                    hipStreamSynchronize(ctx->stream) == hipSuccess;
+    if (!ok) (void)hipStreamSynchronize(ctx->stream);
+    ctx->pool.release(side);
+    return ok ? MF_OK : MF_ERR_DEVICE;
+  }
   std::vector<int> h((size_t)G.n);
   HIP_TRY(hipMemcpy(h.data(), G.h, sizeof(int) * G.n, hipMemcpyDeviceToHost));
   // After the final global relabel, h < H exactly on the vertices that reach the sink.
