@@ -90,7 +90,8 @@ typedef struct mf_options {
   int32_t profile_kernels;    /* N > 0: every N-th push-relabel launch carries start/end events in
                                  its dispatch packet (1 = every launch; each timed launch costs a
                                  cache flush, so sample for low overhead) */
-  int32_t bfs_block_frontier; /* frontier size up to which the one-workgroup BFS runs; 0 = default */
+  int32_t bfs_block_frontier; /* frontier size up to which the one-workgroup BFS runs; 0 = default
+                                 (its variant for graphs of low degree: eight times this) */
   float relabel_time_ratio;   /* adaptive cadence: after a global relabel taking T ms, cycles run
                                  for about ratio * T ms; 0 = default (2) */
   int32_t batch_algo;         /* mf_batch_solve: 0 = TC (default), 1 = VC */

@@ -61,7 +61,9 @@ def check(mf, orc, ctx, g):
     (1300, 19),    # about as many vertices as fit with their excesses
     (1301, 20),    # more: excesses in global memory
     (1500, 41),    # nearly as many as fit at all
-    (1600, 42),    # too many
+    (1600, 42),    # too many: on the grid, its global relabels in one workgroup
+    (9000, 8),     # their frontiers handed to grid-wide levels and back
+    (20000, 4),    # frontiers longer than the LDS lists
     (2048, 13), (2049, 13),  # the widest frontiers that stay with excesses in global memory, and wider
     (2800, 8), (2801, 8), (4000, 2),  # and in LDS; two wide frontiers stay
 ])
