@@ -78,3 +78,21 @@ def test_chains(mf, orc, ctx, width, length):
 ])
 def test_hubs(mf, orc, ctx, k, layers):
     check(mf, orc, ctx, dense_layers(mf, k, layers, seed=k))
+
+
+@pytest.mark.parametrize("frontier", [1, 2, 300])
+@pytest.mark.parametrize("direction", [0, 1, 2])
+def test_relabel_takeover(mf, orc, ctx, frontier, direction):
+    # the one-workgroup search takes over behind grid-wide levels, top-down and bottom-up, at the
+    # smallest frontier, at most of them and where only some fit
+    for g in (chains(mf, 200, 420, seed=5), mf.gen_bipartite(40000, 41000, 6.0, 7),
+              mf.gen_rmat(14, 16, seed=3)):
+        value = orc.dinic_maxflow(g)
+        dg = ctx.upload(g, mf.LAYOUT_BCSR)
+        try:
+            r = dg.solve(mf.ALGO_VC, bfs_block_frontier=frontier, bfs_direction=direction)
+            assert r.value == value and 0 <= r.bfs_grid_levels <= r.bfs_levels
+            assert orc.certify(g, dg.read_flow(return_excess=False), value,
+                               preflow=True)[0] == "ok"
+        finally:
+            dg.close()

@@ -1014,6 +1014,8 @@ __global__ void k_bfs_init(BfsArgs a, int *ccnt0, int *ccnt1) {
       a.state[3] = 0;
       a.state[4] = 0;  // slots explored by grid-wide levels (a 64-bit counter in words 4 and 5)
       a.state[5] = 0;
+      a.state[8] = 0;  // top-down and bottom-up grid levels run
+      a.state[9] = 0;
     }
   }
 }
@@ -1085,6 +1087,7 @@ __global__ __launch_bounds__(kBlock) void k_bfs_level(L g, BfsArgs a, Dispatch d
       a.state[2 + ((level + 1) & 1)] = level + 1;  // the next level may run
       // estimated slots of the top-down frontiers expanded so far (the bottom-up rule's input)
       atomicAdd((unsigned long long *)(a.state + 4), (unsigned long long)slots);
+      a.state[8]++;
     }
   }
   if (blockIdx.x == 0 && threadIdx.x < (unsigned)kNumClasses)
@@ -1127,6 +1130,16 @@ __global__ __launch_bounds__(kBlock) void k_bfs_level(L g, BfsArgs a, Dispatch d
 // spin limit sets *abort and every block leaves; the host then redoes the global relabel without
 // cooperative levels.
 
+// Where a one-workgroup kernel starts (level < 0: at the level that the grid-wide levels before it
+// left), and the frontier it takes over.
+struct Takeover {
+  int level;
+  int size;         // at most this many vertices
+  long long slots;  // and estimated slots
+};
+__device__ __forceinline__ int takeover_level(const BfsArgs &a, const Takeover &t) {
+  return t.level >= 0 ? t.level : max(a.state[0], max(a.state[2], a.state[3]));
+}
 struct CoopStop {
   int small;              // back to the one-workgroup kernel at or below this frontier size,
   long long small_slots;  //   this many estimated slots and fitting its LDS groups
@@ -1333,6 +1346,7 @@ __global__ __launch_bounds__(kBlock) void k_bfs_bottom_up(L g, BfsArgs a, Dispat
       a.state[2 + ((level + 1) & 1)] = level + 1;  // the next level may run
       // estimated slots of the frontiers expanded so far (the bottom-up rule's input)
       atomicAdd((unsigned long long *)(a.state + 4), (unsigned long long)slots);
+      a.state[9]++;
     }
   }
   if (blockIdx.x == 0 && threadIdx.x < (unsigned)kNumClasses) {
@@ -1507,7 +1521,7 @@ __device__ __forceinline__ void wg_expand(const L &g, const BfsArgs &a, const Wg
 }
 
 template <class L>
-__global__ __launch_bounds__(kWgBlock) void k_bfs_wg(L g, BfsArgs a, Dispatch d, int level,
+__global__ __launch_bounds__(kWgBlock) void k_bfs_wg(L g, BfsArgs a, Dispatch d, Takeover take,
                                                      int fmax) {
   constexpr bool kPre = L::kSeg == 1;
   __shared__ int s_u[2][kWgCap];
@@ -1521,6 +1535,7 @@ __global__ __launch_bounds__(kWgBlock) void k_bfs_wg(L g, BfsArgs a, Dispatch d,
   const int tid = (int)threadIdx.x;
   long long nv = 0, ns = 0;
   fmax = min(fmax, kWgCap);
+  int level = takeover_level(a, take);
   // take over the current frontier from the device lists if it fits
   ListSet in = a.fr[0];
   in.items = (level & 1) ? a.fr[1].items : a.fr[0].items;
@@ -1543,7 +1558,7 @@ __global__ __launch_bounds__(kWgBlock) void k_bfs_wg(L g, BfsArgs a, Dispatch d,
       n[q] += k;
     }
     s_size = sz;
-    s_go = sz > 0 && sz <= fmax && slots <= a.wg_slots && n[0] <= kWgCapA && n[1] <= kWgCapB &&
+    s_go = sz > 0 && sz <= min(fmax, take.size) && slots <= take.slots && n[0] <= kWgCapA && n[1] <= kWgCapB &&
            n[2] <= kWgCapC;
   }
   __syncthreads();
@@ -1772,7 +1787,7 @@ __device__ __forceinline__ void bits_frontier(const L &g, const BfsArgs &a, cons
 // As k_bfs_wg: takes the device frontier of `level` over if it has at most fmax vertices (and about
 // a.wg_slots slots), runs levels until the frontier is empty or larger, hands it back by class.
 template <class L>
-__global__ __launch_bounds__(kWgBlock) void k_bfs_bits(L g, BfsArgs a, Dispatch d, int level,
+__global__ __launch_bounds__(kWgBlock) void k_bfs_bits(L g, BfsArgs a, Dispatch d, Takeover take,
                                                        int fmax, const int *src, int mean,
                                                        int lds_bytes) {
   extern __shared__ __align__(16) char lds[];
@@ -1787,6 +1802,7 @@ __global__ __launch_bounds__(kWgBlock) void k_bfs_bits(L g, BfsArgs a, Dispatch 
   m.S = &S;
   m.s = src[0];
   fmax = min(fmax, m.cap);
+  int level = takeover_level(a, take);
   ListSet in = a.fr[0];
   in.items = (level & 1) ? a.fr[1].items : a.fr[0].items;
   in.cnt = pick(a.fcnt, level % 3);
@@ -1800,7 +1816,7 @@ __global__ __launch_bounds__(kWgBlock) void k_bfs_bits(L g, BfsArgs a, Dispatch 
       slots += (long long)k * pick(a.cls_mean, c);
     }
     S.size = sz;
-    S.go = sz > 0 && sz <= fmax && slots <= a.wg_slots;
+    S.go = sz > 0 && sz <= min(fmax, take.size) && slots <= take.slots;
     S.over = 0;
   }
   if (tid < 3) S.cnt[tid] = 0;
@@ -2727,7 +2743,9 @@ enum {
   CTL_FLAGS = CTL_CCNT + 3 * kNumClasses * kCtlStride, // [0] source reached, [1] list overflow
   CTL_STATE = CTL_FLAGS + kCtlStride,                  // [0] level, [1] frontier size,
                                                        // [2..3] grid levels' marks,
-                                                       // [4..5] slots explored
+                                                       // [4..5] slots explored,
+                                                       // [6..7] grid barrier, its failure
+                                                       // [8..9] grid levels run
   CTL_RCNT = CTL_STATE + kCtlStride,                   // 3 x kNumClasses unreached-list counters
   CTL_READ = CTL_RCNT,                                 // the part the host reads back
   CTL_SIZE = CTL_RCNT + 3 * kNumClasses * kCtlStride
@@ -3381,7 +3399,7 @@ static mf_status run_solve(mf_context *ctx, DevGraph &G, const L &lay, mf_algo a
   relabel_again:
     k_bfs_init<<<vgrid, 256, 0, st>>>(ba, ccnt[0], ccnt[1]);
     k_bfs_seed<<<kgrid, 256, 0, st>>>(ba, G.src, G.snk, G.k);
-    int level = 0, levels_total = 0;
+    int level = 0, levels_total = 0, bu_run = 0;
     auto frontier_slots = [&](int lv) {
       double sl = 0;
       for (int c = 0; c < bcfg.nclass; ++c)
@@ -3396,12 +3414,22 @@ static mf_status run_solve(mf_context *ctx, DevGraph &G, const L &lay, mf_algo a
         grp[wg_group(c)] += hstate[ctl_cnt(CTL_FCNT, lv % 3, c)];
       return grp[0] <= kWgCapA && grp[1] <= kWgCapB && grp[2] <= kWgCapC;
     };
-    for (;;) {
+    auto one_workgroup = [&](const Takeover &take) {
       if (use_bits)
-        k_bfs_bits<L><<<1, kWgBlock, bits_lds, st>>>(lay, ba, bdisp, level, fmax, G.src, bits_mean,
+        k_bfs_bits<L><<<1, kWgBlock, bits_lds, st>>>(lay, ba, bdisp, take, fmax, G.src, bits_mean,
                                                      bits_lds);
       else
-        k_bfs_wg<L><<<1, kWgBlock, 0, st>>>(lay, ba, bdisp, level, fmax);
+        k_bfs_wg<L><<<1, kWgBlock, 0, st>>>(lay, ba, bdisp, take, fmax);
+    };
+    // Behind every batch of grid-wide levels, taking over at the sizes at which those levels stop for
+    // it: a read-back between them, about 45 us, costs as much as several levels, a launch that leaves
+    // at once 3.  (40,009 x 39,019 matching 3.53 -> 3.27 ms a solve, R-MAT 13 0.90 -> 0.83, R-MAT 18
+    // 2.29 -> 2.19, R-MAT 20 3.05 -> 2.99.  Grid-wide levels behind the first workgroup kernel in the
+    // same way: matching level, R-MAT 18 2.30, and 20,000 x 60,000 matching 1.02 -> 1.12: they often
+    // find an empty frontier or one that goes bottom-up.)
+    const Takeover behind{-1, fmax_low, ba.wg_slots / 2};
+    for (;;) {
+      one_workgroup(Takeover{level, fmax, ba.wg_slots});
       HIP_TRY(hipGetLastError());
       HIP_TRY(hipMemcpyAsync(hstate, G.ctl, sizeof(int) * CTL_READ, hipMemcpyDeviceToHost, st));
       HIP_TRY(hipStreamSynchronize(st));
@@ -3424,8 +3452,7 @@ static mf_status run_solve(mf_context *ctx, DevGraph &G, const L &lay, mf_algo a
           else if (bottom_up && (int64_t)size * kBottomUpBeta < G.nonzero) bottom_up = false;
         }
         bottom_up = bottom_up || bu_always;
-        int next;
-        bool was_bu = false;
+        bool was_bu = false, coop = false;
         if (bottom_up) {
           // the first bottom-up level of a run walks every vertex; its unreached list, which the
           // next bottom-up level walks, starts empty
@@ -3435,9 +3462,8 @@ static mf_status run_solve(mf_context *ctx, DevGraph &G, const L &lay, mf_algo a
           for (int q = 0; q < kBottomUpBatch; ++q)
             k_bfs_bottom_up<L><<<bugrid, kBlock, 0, st>>>(lay, ba, budisp, G.vo, level + q,
                                                           q == 0 && !bu_prev, level, stay);
-          bu_prev = true;
           was_bu = true;
-          next = -1;
+          one_workgroup(behind);
         } else if (use_coop && mf <= (double)kCoopSlots) {
           // levels inside one cooperative launch until the frontier leaves the mid-size range
           CoopStop cs;
@@ -3454,8 +3480,7 @@ static mf_status run_solve(mf_context *ctx, DevGraph &G, const L &lay, mf_algo a
                           (void *)&cs,  (void *)&bar, (void *)&abort_flag};
           HIP_TRY(hipLaunchCooperativeKernel((const void *)k_bfs_coop<L>, dim3(kCoopBlocks),
                                              dim3(kBlock), args, 0, st));
-          next = -2;
-          bu_prev = false;
+          coop = true;
         } else {
           // top-down levels go kGridLevelBatch at a time between two read-backs; the levels after
           // the first stop by themselves (LevelStop) when the frontier empties, nears half the
@@ -3470,26 +3495,26 @@ static mf_status run_solve(mf_context *ctx, DevGraph &G, const L &lay, mf_algo a
                               : std::numeric_limits<long long>::max();
           for (int q = 0; q < kGridLevelBatch; ++q)
             k_bfs_level<L><<<bgrid, kBlock, 0, st>>>(lay, ba, bdisp, level + q, ls);
-          next = -1;
-          bu_prev = false;
+          one_workgroup(behind);
         }
         HIP_TRY(hipGetLastError());
         HIP_TRY(hipMemcpyAsync(hstate, G.ctl, sizeof(int) * CTL_READ, hipMemcpyDeviceToHost, st));
         HIP_TRY(hipStreamSynchronize(st));
-        if (next == -2) {
-          if (hstate[CTL_STATE + 7] != 0) {  // a grid barrier gave up: redo without them
-            coop_failed = true;
-            break;
-          }
-          next = hstate[CTL_STATE];
+        if (coop && hstate[CTL_STATE + 7] != 0) {  // a grid barrier gave up: redo without them
+          coop_failed = true;
+          break;
         }
-        if (next < 0) next = std::max(hstate[CTL_STATE + 2], hstate[CTL_STATE + 3]);
-        if (was_bu) bfs_bu_levels += next - level;
-        bfs_grid_levels += next - level;
+        const int next = hstate[CTL_STATE];
+        if (coop) bfs_grid_levels += next - level;
+        // the unreached list is the next bottom-up level's if no other level ran behind it
+        bu_prev = was_bu && next - level == hstate[CTL_STATE + 9] - bu_run;
+        bu_run = hstate[CTL_STATE + 9];
         level = next;
         size = 0;
         for (int c = 0; c < bcfg.nclass; ++c) size += hstate[ctl_cnt(CTL_FCNT, level % 3, c)];
-        if (size <= fmax_low && frontier_slots(level) <= ba.wg_slots / 2 && fits_wg(level)) break;
+        if (size == 0) break;
+        // (cooperative levels: no one-workgroup kernel followed)
+        if (coop && size <= fmax_low && frontier_slots(level) <= ba.wg_slots / 2 && fits_wg(level)) break;
       }
       if (coop_failed || size == 0) break;
     }
@@ -3499,6 +3524,8 @@ static mf_status run_solve(mf_context *ctx, DevGraph &G, const L &lay, mf_algo a
     }
     levels_total = level;
     bfs_levels += level;
+    bfs_grid_levels += hstate[CTL_STATE + 8] + hstate[CTL_STATE + 9];
+    bfs_bu_levels += hstate[CTL_STATE + 9];
     HIP_TRY(hipEventRecord(e1, st));
     HIP_TRY(hipEventSynchronize(e1));
     float ms = 0;
