@@ -85,7 +85,8 @@ WORKLOADS = {
 # interleaved).  Started from these options, the autotuner kept them on both graphs (R-MAT 22: 138
 # trials, best 7.42 ms; Genrmf 64: 147 trials, best 93.7 ms).  Genrmf 64's tile widths then
 # narrowed to 4 / 4 / 8 / 16 lanes up to 1,024 slots: 92.0 against 94.7 ms (8 interleaved solves
-# each).  Workloads not listed run the library defaults.
+# each), and 83.5 ms since the one-workgroup levels of low-degree graphs keep their marks in LDS
+# (89.0 with the defaults).  Workloads not listed run the library defaults.
 TUNED = {
     ("rmat22", "vc"): {"cycles_per_relabel": 12, "tile_lanes": 0, "bfs_block_frontier": 1024,
                        "relabel_time_ratio": 2.0, "bfs_direction": 0,
