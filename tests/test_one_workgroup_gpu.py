@@ -96,3 +96,22 @@ def test_relabel_takeover(mf, orc, ctx, frontier, direction):
                                preflow=True)[0] == "ok"
         finally:
             dg.close()
+
+
+def test_threads_of_different_sizes(mf, orc):
+    # graphs that ask for little and for nearly all LDS, solved side by side, a context each
+    from concurrent.futures import ThreadPoolExecutor
+
+    graphs = [chains(mf, 3, 4, 1), chains(mf, 1300, 19, 2), chains(mf, 1500, 41, 3),
+              chains(mf, 2000, 60, 4)]
+    want = [orc.dinic_maxflow(g) for g in graphs]
+
+    def solve(g):
+        ctx = mf.Context(0)
+        try:
+            return [ctx.solve(g).value for _ in range(10)]
+        finally:
+            ctx.close()
+
+    with ThreadPoolExecutor(len(graphs)) as pool:
+        assert list(pool.map(solve, graphs)) == [[v] * 10 for v in want]

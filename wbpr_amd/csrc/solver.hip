@@ -3272,8 +3272,10 @@ static mf_status run_solve(mf_context *ctx, DevGraph &G, const L &lay, mf_algo a
     bits_lds = (int)std::min<int64_t>(marks + 8LL * n, (ctx->lds_limit - kWgStaticLds) & ~15);
     const int64_t cap = std::min<int64_t>(n, (bits_lds - marks) / 8);
     fmax = (int)std::min<int64_t>((int64_t)kBitsFrontier * std::min(fmax, 1 << 20), cap);
+    // (the same value in every thread, whatever its graph's size)
     HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(k_bfs_bits<L>),
-                                hipFuncAttributeMaxDynamicSharedMemorySize, bits_lds));
+                                hipFuncAttributeMaxDynamicSharedMemorySize,
+                                ctx->lds_limit - kWgStaticLds));
   }
   const int fmax_low = std::max(1, fmax / 2);
   bool use_coop = ctx->cooperative && o.bfs_cooperative == 1;

@@ -65,11 +65,13 @@ int wg_single_kind(int32_t n, int lds_limit) {
   return kind == kWgGlobal ? -1 : kind;
 }
 
+// (The attribute is the kernel's, not the launch's: every thread sets the same value, not its own
+// launch's size, which another thread's smaller graph could lower before the launch.)
 template <class L, int KIND>
-static hipError_t launch_single(hipStream_t st, const L &g, const WgSingle &a) {
+static hipError_t launch_single(hipStream_t st, const L &g, const WgSingle &a, int lds_limit) {
   const hipError_t e =
       hipFuncSetAttribute(reinterpret_cast<const void *>(k_wg_solve<L, KIND>),
-                          hipFuncAttributeMaxDynamicSharedMemorySize, a.lds_bytes);
+                          hipFuncAttributeMaxDynamicSharedMemorySize, lds_limit - kWgStaticLds);
   if (e != hipSuccess) return e;
   k_wg_solve<L, KIND><<<1, kWgThreads, a.lds_bytes, st>>>(g, a);
   return hipGetLastError();
@@ -79,8 +81,8 @@ template <class L>
 hipError_t wg_single_launch(hipStream_t st, const L &g, WgSingle a, int kind, int lds_limit) {
   const long long all = wg_state_bytes(kind, a.n) + 2LL * wg_item_bytes(kind) * a.n;
   a.lds_bytes = (int)std::min<long long>((all + 15) / 16 * 16, lds_limit - kWgStaticLds);
-  return kind == kWgBoth ? launch_single<L, kWgBoth>(st, g, a)
-                         : launch_single<L, kWgHeights>(st, g, a);
+  return kind == kWgBoth ? launch_single<L, kWgBoth>(st, g, a, lds_limit)
+                         : launch_single<L, kWgHeights>(st, g, a, lds_limit);
 }
 template hipError_t wg_single_launch(hipStream_t, const LayoutBCSR &, WgSingle, int, int);
 template hipError_t wg_single_launch(hipStream_t, const LayoutBCSR2 &, WgSingle, int, int);
