@@ -6,13 +6,15 @@
 // list by size instead and are used again; at most `limit` bytes are kept, larger blocks and
 // what is beyond the limit are given back at once, the rest with the context.  A context
 // belongs to one host thread at a time, and its calls end with their stream idle: a block on the
-// list has no work in flight.
+// list has no work in flight.  The lock is for handles that another thread destroys (a garbage
+// collector's), as hipFree allowed.
 #pragma once
 
 #include <hip/hip_runtime.h>
 
 #include <cstddef>
 #include <map>
+#include <mutex>
 #include <unordered_map>
 #include <vector>
 
@@ -24,6 +26,7 @@ class DevPool {
 
   hipError_t alloc(void **p, size_t bytes) {
     const size_t size = rounded(bytes);
+    std::lock_guard<std::mutex> lock(mutex_);
     auto it = kept_.find(size);
     if (it != kept_.end() && !it->second.empty()) {
       *p = it->second.back();
@@ -34,7 +37,7 @@ class DevPool {
     hipError_t e = hipMalloc(p, size);
     if (e == hipErrorOutOfMemory && kept_bytes_ > 0) {
       (void)hipGetLastError();
-      trim();
+      trim_locked();
       e = hipMalloc(p, size);
     }
     if (e == hipSuccess) size_[*p] = size;
@@ -43,6 +46,7 @@ class DevPool {
 
   // p: from alloc, with no device work on it in flight.
   void release(void *p) {
+    std::lock_guard<std::mutex> lock(mutex_);
     const auto it = size_.find(p);
     if (it != size_.end() && it->second <= kMaxBlock && kept_bytes_ + it->second <= limit) {
       kept_[it->second].push_back(p);
@@ -54,6 +58,12 @@ class DevPool {
   }
 
   void trim() {
+    std::lock_guard<std::mutex> lock(mutex_);
+    trim_locked();
+  }
+
+ private:
+  void trim_locked() {
     for (auto &q : kept_)
       for (void *p : q.second) {
         size_.erase(p);
@@ -63,7 +73,6 @@ class DevPool {
     kept_bytes_ = 0;
   }
 
- private:
   static constexpr size_t kMaxBlock = size_t(32) << 20;
 
   // Up to an eighth more, so that graphs of about one size share blocks.
@@ -74,6 +83,7 @@ class DevPool {
     return (bytes + step - 1) / step * step;
   }
 
+  std::mutex mutex_;
   std::map<size_t, std::vector<void *>> kept_;
   std::unordered_map<void *, size_t> size_;
   size_t kept_bytes_ = 0;
