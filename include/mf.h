@@ -354,7 +354,9 @@ typedef struct mf_server_times {
 } mf_server_times;
 mf_status mf_server_create(mf_context *ctx, int64_t hbm_budget_bytes, int32_t max_inflight_launches,
                            mf_server **out);
-/* Submit a request; *request_id receives its id.  MF_ERR_BUDGET if it can never fit. */
+/* Submit a request; *request_id receives its id.  MF_ERR_BUDGET if it can never fit; MF_ERR_OVERFLOW
+ * (requests of the serving kernel; one that runs alone fails when it is solved) if the source's arcs
+ * hold more than an int32 of capacity -- in the serving kernel only if the sink's do too. */
 mf_status mf_server_submit(mf_server *srv, const mf_csr *g, int64_t *request_id);
 /* Advance the loop: collect finished requests, admit what fits, publish finished copies into
  * the running batch, launch the serving kernel again if no workgroup of it is left.

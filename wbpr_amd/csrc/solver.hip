@@ -4101,13 +4101,15 @@ mf_status serve_prepare(const mf_csr *g, ServeInstance &I) {
   I.n = g->n;
   I.S = L.slots;
   // a value is all a request returns: with clearly less capacity into t than out of s the reversed
-  // network is laid out (see pack_instances)
+  // network is laid out (see pack_instances), and also where only the capacity into t is an int32
+  // -- no excess is larger than the capacity it started from
   int64_t from_s = 0, into_t = 0;
   for (int32_t j = L.off[(size_t)g->s]; j < L.off[(size_t)g->s + 1]; ++j)
     if (L.dst[(size_t)j] != g->s) from_s += L.cap0[(size_t)j];
   for (int32_t j = L.off[(size_t)g->t]; j < L.off[(size_t)g->t + 1]; ++j)
     if (L.dst[(size_t)j] != g->t) into_t += L.cap0[(size_t)L.rev[(size_t)j]];
-  const bool reverse = solves_reversed(from_s, into_t);
+  const bool reverse = solves_reversed(from_s, into_t) || from_s > INT32_MAX;
+  if ((reverse ? into_t : from_s) > INT32_MAX) return MF_ERR_OVERFLOW;
   I.s = reverse ? g->t : g->s;
   I.t = reverse ? g->s : g->t;
   I.off = std::move(L.off);
