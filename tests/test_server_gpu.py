@@ -35,3 +35,32 @@ def test_more_than_an_int32_out_of_the_source(mf, ctx, into_t, value):
             assert serve(srv, [srv.submit(g)]) == [value]
     finally:
         srv.close()
+
+
+def beside_backlog(mf, orc, ctx, big, budget=4 << 30):
+    """For each of four requests that run alone: how many of 600 small ones of 13 to 22 ms each,
+    published before it, were unfinished when it had its result."""
+    small = mf.gen_genrmf(16, 60, 1, 10000, 3)
+    srv = mf.Server(ctx, hbm_budget_bytes=budget, max_inflight_launches=4)
+    try:
+        first = [srv.submit(small) for _ in range(600)]
+        t0 = time.time()
+        while srv.stats()["admitted"] < len(first) and time.time() - t0 < 60:
+            srv.progress()
+        alone = [srv.submit(big) for _ in range(4)]
+        values = serve(srv, first + alone)
+        assert set(values[:600]) == {orc.dinic_maxflow(small)}
+        assert set(values[600:]) == {orc.dinic_maxflow(big)}
+        assert [srv.times(i)["batched"] for i in alone] == [0] * 4
+        ends = np.array([srv.times(i)["finish_ms"] for i in first])
+        return [int((ends > srv.times(i)["finish_ms"]).sum()) for i in alone]
+    finally:
+        srv.close()
+
+
+@pytest.mark.parametrize("gen,args", [("gen_genrmf", (20, 45, 1, 10000, 5)),    # in one workgroup
+                                      ("gen_bipartite", (20000, 15000, 8.0, 77))])  # on the grid
+def test_large_request_beside_a_backlog(mf, orc, ctx, gen, args):
+    # more small requests than there are CUs are queued: a large one does not wait for them to
+    # leave the serving kernel
+    assert max(beside_backlog(mf, orc, ctx, getattr(mf, gen)(*args))) >= 256

@@ -404,7 +404,8 @@ mf_status mf_server_create(mf_context *ctx, int64_t hbm_budget_bytes, int32_t ma
   srv->arena_nv = std::min<int64_t>(srv->arena_nv, (INT32_MAX / 4) - 1);
   srv->arena_ns = std::min<int64_t>(srv->arena_nv * kSlotsPerVertex, INT32_MAX - 1);
   if (srv->arena_nv < 2) return MF_ERR_BUDGET;
-  mf_status s = serve_arena_create(ctx, srv->arena_nv, srv->arena_ns, kQueueCap, &srv->arena);
+  mf_status s = serve_arena_create(ctx, srv->arena_nv, srv->arena_ns, kQueueCap, max_inflight_launches,
+                                   &srv->arena);
   if (s != MF_OK) return s;
   srv->vranges = Ranges(srv->arena_nv);
   srv->sranges = Ranges(srv->arena_ns);

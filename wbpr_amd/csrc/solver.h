@@ -90,7 +90,8 @@ mf_status serve_prepare(const mf_csr *g, ServeInstance &inst);
 // Device bytes of an arena of nv vertices and ns slots (an instance takes n + 1 vertices and
 // 2m slots).
 int64_t serve_arena_bytes(int64_t nv, int64_t ns);
-mf_status serve_arena_create(mf_context *ctx, int64_t nv, int64_t ns, int32_t qcap,
+// alone: solves that may run beside the serving kernel at a time, which leaves CUs for them.
+mf_status serve_arena_create(mf_context *ctx, int64_t nv, int64_t ns, int32_t qcap, int32_t alone,
                              ServeArena **out);
 // Leaves idle workgroups, waits for the kernel and the copies, frees everything.
 void serve_arena_destroy(ServeArena *a);

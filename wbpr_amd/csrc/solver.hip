@@ -3993,17 +3993,26 @@ void batch_release(BatchResident *r) {
 
 // ---- serving arena (host side of k_serve_wg) ---------------------------------------------------
 
-constexpr int kServeGroupsPerCU = 1;               // resident serving workgroups per CU
-// LDS of a serving workgroup: the state of the largest instance and its lists.  The rest of a CU's
-// 160 KB stays with the solves that run alone beside it.
+// LDS of a serving workgroup: the state of the largest instance and its lists.  One fits a CU, and
+// beside it no one-workgroup kernel of a solve that runs alone (k_wg_solve and k_bfs_bits ask for up
+// to 156 KB, k_bfs_wg has 56 KB): the serving grid leaves CUs free for those (serve_groups).
 constexpr int kServeLds = 112 << 10;
 static_assert(wg_kind(kServeVertices, kServeLds) == kWgBoth, "every served instance fits");
+constexpr int kXcds = 8;
+// Workgroups of the serving kernel: one to a CU, but for as many CUs of every XCD as solves may run
+// alone at a time.  A solve has one such kernel in flight, and the only workgroup of a launch always
+// goes to the first XCD, as workgroup i does to XCD i mod 8.  (With a workgroup on every CU a request
+// of 18,000 vertices waited for 42 to 64 ms beside 600 of 13 to 22 ms, whatever the queue held last.)
+static int serve_groups(int num_cu, int alone) {
+  return std::max(num_cu / 2, num_cu - kXcds * alone);
+}
 constexpr long long kServeIdleTicks = 200000;      // 2 ms at the 100 MHz wall clock
 
 struct ServeArena {
   mf_context *ctx = nullptr;
   int64_t nv = 0, ns = 0;  // vertex and slot capacity
   int32_t qcap = 0;
+  int groups = 1;          // workgroups of the serving kernel
   // device arena
   int *off = nullptr, *rev = nullptr, *h = nullptr, *e = nullptr, *stamp = nullptr;
   int *lists = nullptr;
@@ -4044,7 +4053,7 @@ int64_t serve_arena_bytes(int64_t nv, int64_t ns) {
   return 33 * nv + 12 * ns;
 }
 
-mf_status serve_arena_create(mf_context *ctx, int64_t nv, int64_t ns, int32_t qcap,
+mf_status serve_arena_create(mf_context *ctx, int64_t nv, int64_t ns, int32_t qcap, int32_t alone,
                              ServeArena **out) {
   if (!ctx || !out || nv <= 0 || ns <= 0 || qcap <= 0 || nv >= INT32_MAX / 4 || ns >= INT32_MAX)
     return MF_ERR_INVALID_ARGUMENT;
@@ -4055,6 +4064,7 @@ mf_status serve_arena_create(mf_context *ctx, int64_t nv, int64_t ns, int32_t qc
   a->nv = nv;
   a->ns = ns;
   a->qcap = qcap;
+  a->groups = serve_groups(ctx->num_cu, alone);
   mf_status rc = MF_OK;
   auto fail = [&](mf_status r) {
     serve_arena_destroy(a);
@@ -4255,8 +4265,7 @@ mf_status serve_launch(ServeArena *a) {
   sa.wide = kWgWideBoth;
   HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(k_serve_wg<LayoutBCSR>),
                               hipFuncAttributeMaxDynamicSharedMemorySize, kServeLds));
-  const int nwg = std::max(1, kServeGroupsPerCU * a->ctx->num_cu);
-  k_serve_wg<LayoutBCSR><<<nwg, kBlock, kServeLds, a->kernel_stream>>>(
+  k_serve_wg<LayoutBCSR><<<a->groups, kBlock, kServeLds, a->kernel_stream>>>(
       LayoutBCSR{a->off, a->dc, a->rev, nullptr}, sa);
   HIP_TRY(hipGetLastError());
   a->launched = true;
