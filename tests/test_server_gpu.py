@@ -64,3 +64,18 @@ def test_large_request_beside_a_backlog(mf, orc, ctx, gen, args):
     # more small requests than there are CUs are queued: a large one does not wait for them to
     # leave the serving kernel
     assert max(beside_backlog(mf, orc, ctx, getattr(mf, gen)(*args))) >= 256
+
+
+@pytest.mark.parametrize("scale,factor", [(13, 16), (14, 4), (14, 15)])
+def test_power_law_requests(mf, orc, ctx, scale, factor):
+    # frontiers wider than 2,800 vertices and hubs: solved with the vertex state in LDS all the same.
+    # One lane for a hub's whole scan took 30 to 100 ms; 20 is well above the 5 to 18 of a wave
+    graphs = [mf.gen_rmat(scale, factor, seed=40 + i) for i in range(4)]
+    srv = mf.Server(ctx, hbm_budget_bytes=1 << 30, max_inflight_launches=1)
+    try:
+        ids = [srv.submit(g) for g in graphs]
+        assert serve(srv, ids) == [orc.dinic_maxflow(g) for g in graphs]
+        assert all(srv.times(i)["batched"] == 1 for i in ids)
+        assert min(srv.times(i)["device_ms"] for i in ids) < 20
+    finally:
+        srv.close()

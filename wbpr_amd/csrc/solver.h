@@ -78,9 +78,9 @@ void batch_release(BatchResident *r);
 struct ServeArena;
 constexpr int32_t kServeVertices = 16384;  // vertices of a served instance, at most
 // A request laid out for the arena on the host: BCSR slots with its own ids (offsets n+1, {dst,
-// capacity} pairs, reverse slots), vertex BFS classes and the class populations.
+// capacity} pairs, reverse slots), vertex BFS classes and the class populations.  wide: see ServeEntry.
 struct ServeInstance {
-  int32_t n = 0, s = 0, t = 0;
+  int32_t n = 0, s = 0, t = 0, wide = 0;
   int64_t S = 0;
   std::vector<int32_t> off, dc, rev;
   std::vector<unsigned char> vcls;

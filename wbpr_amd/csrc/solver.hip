@@ -2325,10 +2325,11 @@ __global__ __launch_bounds__(kBlock) void k_batch_wg(L g, BatchArgs b) {
 
 struct ServeEntry {
   int vb, sb, n, s, t;    // first vertex and slot in the arena, vertices, source, sink (local ids)
+  int wide;               // > 0: a frontier wider than this goes to batch_instance
   int pop[kNumClasses];   // cycle-class populations of the instance
   int bpop[kNumClasses];  // BFS-class populations
 };
-constexpr int kServeEntryInts = 5 + 2 * kNumClasses;
+constexpr int kServeEntryInts = 6 + 2 * kNumClasses;
 static_assert(sizeof(ServeEntry) == sizeof(int) * kServeEntryInts, "ServeEntry is plain ints");
 
 struct ServeReport {
@@ -2352,7 +2353,6 @@ struct ServeArgs {
   int qcap;
   int lds_bytes;               // dynamic LDS of a workgroup
   float wg_ratio;              // cycle time / relabel time of the LDS solver
-  int wide;                    // frontiers wider than this take batch_instance
   long long idle_ticks;        // ticks without any claim or finish after which idle workgroups
                                // leave (none may be busy)
 };
@@ -2451,7 +2451,7 @@ __global__ __launch_bounds__(kBlock) void k_serve_wg(L g, ServeArgs a) {
       WgSolver<LayoutBCSR, kWgBoth, kBlock> w{gi, s_wg, 0, n, s_entry[3], s_entry[4]};
       w.st = WgStats{0, 0, 0, 0, 0, 0};
       w.carve(lds, a.lds_bytes, nullptr, nullptr);
-      const WgOutcome o = w.solve(a.wg_ratio, a.b.max_cycles, a.b.max_rounds, a.wide, 0);
+      const WgOutcome o = w.solve(a.wg_ratio, a.b.max_cycles, a.b.max_rounds, s_entry[5], 0);
       value = o.value;
       status = o.status;
       st = Stats{w.st.active, w.st.slots, w.st.pushes, w.st.relabels};
@@ -2471,7 +2471,7 @@ __global__ __launch_bounds__(kBlock) void k_serve_wg(L g, ServeArgs a) {
         b.stamp[v] = -1;
       }
       __syncthreads();
-      const BatchInst I{0, n, s_entry[3], s_entry[4], s_entry + 5, s_entry + 5 + kNumClasses};
+      const BatchInst I{0, n, s_entry[3], s_entry[4], s_entry + 6, s_entry + 6 + kNumClasses};
       value = batch_instance(gi, b, I, &status, s_f, s_c, s_flag, &s_dec, s_tab, st, nv, ns);
     }
     // every write of the instance reaches memory before the host may reuse its ranges
@@ -4131,12 +4131,19 @@ mf_status serve_prepare(const mf_csr *g, ServeInstance &I) {
   I.rev = std::move(L.rev);
   I.vcls.resize((size_t)I.n);
   for (int q = 0; q < kNumClasses; ++q) I.pop[q] = I.bpop[q] = 0;
+  int64_t heavy = 0;
   for (int32_t v = 0; v < I.n; ++v) {
     const int c = class_of_degree(vc, (int64_t)(I.off[(size_t)v + 1] - I.off[(size_t)v]));
     I.vcls[(size_t)v] = (unsigned char)c;
     I.bpop[c]++;
+    if (c >= kHeavyClass && v != g->s && v != g->t)
+      heavy += I.off[(size_t)v + 1] - I.off[(size_t)v];
   }
   I.pop[0] = I.n;  // thread-centric cycles: one class
+  // Only requests of low degree (low_degree's rule) give the LDS solver up on a wide frontier: a hub is
+  // a wave's step there, a lane's whole scan in batch_instance's thread-centric cycles.  (R-MAT 13, edge
+  // factor 16: 48 ms of device time there, 3.9 ms with LDS; R-MAT 12 to 14, edge factor 8: 25 and 3.5.)
+  I.wide = heavy * 8 <= I.S ? kWgWideBoth : 0;
   return MF_OK;
 }
 
@@ -4176,7 +4183,7 @@ void serve_copy_release(void *done) {
 
 void serve_publish(ServeArena *a, int64_t q, const ServeInstance &I, int32_t vb, int64_t sb) {
   int *en = a->entries + (size_t)(q % a->qcap) * kServeEntryInts;
-  const int vals[kServeEntryInts] = {vb, (int)sb, I.n, I.s, I.t,
+  const int vals[kServeEntryInts] = {vb, (int)sb, I.n, I.s, I.t, I.wide,
                                      I.pop[0], I.pop[1], I.pop[2], I.pop[3], I.pop[4], I.pop[5],
                                      I.bpop[0], I.bpop[1], I.bpop[2], I.bpop[3], I.bpop[4],
                                      I.bpop[5]};
@@ -4262,7 +4269,6 @@ mf_status serve_launch(ServeArena *a) {
   sa.idle_ticks = kServeIdleTicks;
   sa.lds_bytes = kServeLds;
   sa.wg_ratio = kDefaultRelabelRatio;
-  sa.wide = kWgWideBoth;
   HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(k_serve_wg<LayoutBCSR>),
                               hipFuncAttributeMaxDynamicSharedMemorySize, kServeLds));
   k_serve_wg<LayoutBCSR><<<a->groups, kBlock, kServeLds, a->kernel_stream>>>(
