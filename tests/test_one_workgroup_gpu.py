@@ -115,3 +115,27 @@ def test_threads_of_different_sizes(mf, orc):
 
     with ThreadPoolExecutor(len(graphs)) as pool:
         assert list(pool.map(solve, graphs)) == [[v] * 10 for v in want]
+
+
+@pytest.mark.parametrize("coop", [0, 1])
+@pytest.mark.parametrize("width,length", [
+    (2801, 8),    # abandoned at the third wide frontier
+    (2049, 13),   # at the first one, level 1
+    (9000, 6),    # a frontier longer than the LDS list
+    (0, 0),       # a matching: the sink's neighbours
+])
+def test_grid_goes_on_from_an_abandoned_search(mf, orc, ctx, width, length, coop):
+    g = chains(mf, width, length, seed=9) if width else mf.gen_bipartite(17000, 16500, 8.0, seed=9)
+    value = orc.dinic_maxflow(g)
+    for layout in (mf.LAYOUT_BCSR, mf.LAYOUT_BCSR2, mf.LAYOUT_RCSR):
+        dg = ctx.upload(g, layout)
+        try:
+            for algo in (mf.ALGO_VC, mf.ALGO_TC):
+                r = dg.solve(algo, bfs_cooperative=coop)
+                assert r.value == value and r.bfs_levels > 0
+                assert coop or r.bfs_grid_levels > 0  # (else its frontier's own level at least)
+                assert orc.certify(g, dg.read_flow(return_excess=False), value,
+                                   preflow=True)[0] == "ok"
+        finally:
+            dg.close()
+    assert ctx.solve_noalloc(g, mf.ALGO_VC, bfs_cooperative=coop).value == value

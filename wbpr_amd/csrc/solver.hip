@@ -1033,6 +1033,24 @@ __global__ void k_bfs_seed(BfsArgs a, const int *src, const int *snk, int k) {
   }
 }
 
+// A first global relabel that k_wg_solve abandoned at `level` goes on from there: the heights are in
+// a.h, that level's vertices become the frontier, the reached ones with excess the worklist.
+__global__ __launch_bounds__(kBlock) void k_bfs_resume(BfsArgs a, int level) {
+  __shared__ Stage sf, sa;
+  stage_init(sf);
+  stage_init(sa);
+  ListSet out = a.fr[0];
+  out.items = (level & 1) ? a.fr[1].items : a.fr[0].items;
+  out.cnt = pick(a.fcnt, level % 3);
+  const int stride = gridDim.x * blockDim.x;
+  for (int v = blockIdx.x * blockDim.x + threadIdx.x; v < a.H; v += stride) {
+    const int h = a.h[v];
+    bfs_append(BfsStages{&sf, &sa}, a, out, v, h == level, h > 0 && h < a.H && a.e[v] > 0);
+  }
+  stage_flush(sf, out, a.nclass);
+  stage_flush(sa, a.active, a.nclass_act);
+}
+
 // LDS frontier entries per group of the one-workgroup BFS (below), by degree class
 constexpr int kWgCapA = 2048, kWgCapB = 256, kWgCapC = 32;
 constexpr int kWgCap = kWgCapA + kWgCapB + kWgCapC;
@@ -3073,11 +3091,20 @@ static bool wg_allowed(const mf_options &o) {
          o.bfs_direction == 0;
 }
 
-// *taken: the solve is done (its status is returned); otherwise nothing has changed but the
-// residuals, which hold the capacities.
+// The first global relabel of a solve as run_one_workgroup left it: abandoned at `level` (0: not
+// begun).  Then the residuals hold the capacities, the excesses are zero and the heights up to that
+// level are on the device, and the grid goes on from there: a search thrown away cost matchings of
+// 17,000 to 30,000 vertices a side 3% of their 2 ms.
+struct FirstRelabel {
+  int level = 0;
+  double t0 = 0, ms = 0;  // when the solve began; device time of the search so far
+  int64_t verts = 0, slots = 0;
+};
+
+// *taken: the solve is done (its status is returned); otherwise see FirstRelabel.
 template <class L>
 static mf_status run_one_workgroup(mf_context *ctx, DevGraph &G, const L &lay, const mf_options &o,
-                                   mf_result *res, bool *taken) {
+                                   mf_result *res, bool *taken, FirstRelabel *first) {
   *taken = false;
   const int64_t slots = 2 * G.m;  // (whatever the layout)
   if (G.k != 1 || !wg_allowed(o) || slots > kWgMaxSlots ||
@@ -3115,7 +3142,10 @@ static mf_status run_one_workgroup(mf_context *ctx, DevGraph &G, const L &lay, c
   HIP_TRY(hipMemcpyAsync(&r, G.ctl, sizeof(r), hipMemcpyDeviceToHost, st));
   HIP_TRY(hipStreamSynchronize(st));
   const double t1 = now_ms();
-  if (r.status == 3) return MF_OK;
+  if (r.status == 3) {
+    *first = FirstRelabel{r.levels, t0, (double)r.t_relabel * 1e-5, r.bfs_verts, r.bfs_slots};
+    return MF_OK;
+  }
   *taken = true;
   G.fresh = false;
   const mf_status status = r.status == 0 ? MF_OK
@@ -3147,7 +3177,8 @@ template <class L>
 static mf_status run_solve(mf_context *ctx, DevGraph &G, const L &lay, mf_algo algo,
                            const mf_options &o, mf_result *res) {
   bool taken = false;
-  const mf_status one = run_one_workgroup(ctx, G, lay, o, res, &taken);
+  FirstRelabel first;
+  const mf_status one = run_one_workgroup(ctx, G, lay, o, res, &taken, &first);
   if (taken || one != MF_OK) return one;
   hipStream_t st = ctx->stream;
   const int n = G.n;
@@ -3340,13 +3371,15 @@ static mf_status run_solve(mf_context *ctx, DevGraph &G, const L &lay, mf_algo a
     for (size_t q = old; q < ctx->prof_ev.size(); ++q) HIP_TRY(hipEventCreate(&ctx->prof_ev[q]));
   }
 
-  const double t0 = now_ms();
-  const int rgrid = std::max(1, (int)std::min<int64_t>((G.S + 255) / 256, 16 * ctx->num_cu));
-  restore_residuals(ctx, G);
+  const double t0 = first.level ? first.t0 : now_ms();
+  if (!first.level) {
+    const int rgrid = std::max(1, (int)std::min<int64_t>((G.S + 255) / 256, 16 * ctx->num_cu));
+    restore_residuals(ctx, G);
+    k_reset_vertices<<<rgrid, 256, 0, st>>>(G.h, G.e, G.stamp, n,
+                                            G.layout == MF_LAYOUT_RCSR ? G.bcf : nullptr,
+                                            G.m);
+  }
   G.fresh = false;
-  k_reset_vertices<<<rgrid, 256, 0, st>>>(G.h, G.e, G.stamp, n,
-                                          G.layout == MF_LAYOUT_RCSR ? G.bcf : nullptr,
-                                          G.m);
   HIP_TRY(hipMemsetAsync(G.stats, 0, sizeof(unsigned long long) * kStatSlot * kStatSpread, st));
   HIP_TRY(hipMemsetAsync(G.ctl, 0, sizeof(int) * CTL_SIZE, st));
   const int pgrid = (int)std::min<int64_t>(16 * ctx->num_cu,
@@ -3354,7 +3387,7 @@ static mf_status run_solve(mf_context *ctx, DevGraph &G, const L &lay, mf_algo a
   k_preflow<L><<<pgrid, kBlock, 0, st>>>(lay, G.e, G.src, G.k, G.stats);
   HIP_TRY(hipGetLastError());
 
-  int hstate[CTL_SIZE];
+  int hstate[CTL_SIZE] = {0};
   // elapsed times of a cycle chunk's timed launches (half: which set of profiling events)
   auto collect = [&](int half, int count) -> hipError_t {
     for (int q = 0; q < count; ++q) {
@@ -3399,9 +3432,19 @@ static mf_status run_solve(mf_context *ctx, DevGraph &G, const L &lay, mf_algo a
     HIP_TRY(hipEventRecord(e0, st));
     bool coop_failed = false;
   relabel_again:
-    k_bfs_init<<<vgrid, 256, 0, st>>>(ba, ccnt[0], ccnt[1]);
-    k_bfs_seed<<<kgrid, 256, 0, st>>>(ba, G.src, G.snk, G.k);
     int level = 0, levels_total = 0, bu_run = 0;
+    // the frontier is known to be wide: grid-wide levels next (cooperative ones need its read-back)
+    bool resumed = rounds == 0 && first.level && !use_coop;
+    if (rounds == 0 && first.level && !coop_failed) {
+      level = first.level;
+      relabel_ms = first.ms;
+      k_bfs_resume<<<std::max(1, std::min((n + kBlock - 1) / kBlock, ctx->num_cu)), kBlock, 0, st>>>(
+          ba, level);
+    } else {
+      resumed = false;
+      k_bfs_init<<<vgrid, 256, 0, st>>>(ba, ccnt[0], ccnt[1]);
+      k_bfs_seed<<<kgrid, 256, 0, st>>>(ba, G.src, G.snk, G.k);
+    }
     auto frontier_slots = [&](int lv) {
       double sl = 0;
       for (int c = 0; c < bcfg.nclass; ++c)
@@ -3430,17 +3473,17 @@ static mf_status run_solve(mf_context *ctx, DevGraph &G, const L &lay, mf_algo a
     // same way: matching level, R-MAT 18 2.30, and 20,000 x 60,000 matching 1.02 -> 1.12: they often
     // find an empty frontier or one that goes bottom-up.)
     const Takeover behind{-1, fmax_low, ba.wg_slots / 2};
-    for (;;) {
-      one_workgroup(Takeover{level, fmax, ba.wg_slots});
-      HIP_TRY(hipGetLastError());
-      HIP_TRY(hipMemcpyAsync(hstate, G.ctl, sizeof(int) * CTL_READ, hipMemcpyDeviceToHost, st));
-      HIP_TRY(hipStreamSynchronize(st));
-      {
+    for (;; resumed = false) {
+      if (!resumed) {
+        one_workgroup(Takeover{level, fmax, ba.wg_slots});
+        HIP_TRY(hipGetLastError());
+        HIP_TRY(hipMemcpyAsync(hstate, G.ctl, sizeof(int) * CTL_READ, hipMemcpyDeviceToHost, st));
+        HIP_TRY(hipStreamSynchronize(st));
         const mf_status fs = finish_cycles();  // the cycles before this relabel have finished
         if (fs != MF_OK) return fs;
+        level = hstate[CTL_STATE];
       }
-      level = hstate[CTL_STATE];
-      int size = hstate[CTL_STATE + 1];
+      int size = resumed ? 1 : hstate[CTL_STATE + 1];
       if (size == 0) break;
       bool bottom_up = false, bu_prev = false;
       for (;;) {  // frontier too large for one workgroup: grid launches per level
@@ -3533,7 +3576,7 @@ static mf_status run_solve(mf_context *ctx, DevGraph &G, const L &lay, mf_algo a
     float ms = 0;
     HIP_TRY(hipEventElapsedTime(&ms, e0, e1));
     relabel_ms += ms;
-    last_relabel_ms = ms;
+    last_relabel_ms = rounds == 0 ? relabel_ms : ms;
     ++rounds;
     if (hstate[CTL_FLAGS] != 0 || hstate[CTL_FLAGS + 1] != 0) {
       status = MF_ERR_INTERNAL;  // residual path from a source, or a worklist overflow
@@ -3670,6 +3713,8 @@ static mf_status run_solve(mf_context *ctx, DevGraph &G, const L &lay, mf_algo a
   long long v0 = 0;
   HIP_TRY(hipMemcpy(&v0, G.values, sizeof(long long), hipMemcpyDeviceToHost));
   HIP_TRY(read_stats(G.stats, hs));
+  hs[ST_BFS_VERTS] += (unsigned long long)first.verts;
+  hs[ST_BFS_SLOTS] += (unsigned long long)first.slots;
   if (res) {
     memset(res, 0, sizeof(*res));
     res->value = v0;

@@ -72,7 +72,8 @@ struct WgStats {
 // What one solve did and how it ended.
 struct WgOutcome {
   long long value;
-  int status;  // 0 ok, 1 round limit, 2 a source was reached (invariant broken), 3 too wide
+  int status;  // 0 ok, 1 round limit, 2 a source was reached (invariant broken), 3 too wide: the
+               // vertices up to `levels` have their heights, the others n
   int rounds, cycles, levels;
   long long source_out;         // this thread's part of the preflow
   long long t_relabel, t_cycle;  // wall_clock64 ticks
@@ -481,8 +482,9 @@ struct WgSolver {
   }
 
   // Heights from a BFS over reverse residual arcs: distances to the sink, n where it cannot be
-  // reached.  Returns the levels; wide > 0 gives up (-1) once more than wide_levels frontiers held
-  // more vertices than that, before anything outside LDS has been written.
+  // reached.  Returns the levels; wide > 0 gives up once more than wide_levels frontiers held more
+  // vertices than that, before anything outside LDS has been written: -1 - level, the heights up to
+  // that level set.
   __device__ __forceinline__ int relabel(int wide, int wide_levels, bool check) {
     const int tid = (int)threadIdx.x;
     for (int v = tid; v < n; v += BS) h[v] = (HT)(v == s ? n + 1 : (v == t ? 0 : n));
@@ -505,7 +507,7 @@ struct WgSolver {
     for (;; ++level) {
       const int cnt = S.cnt[level % 3];
       if (cnt == 0) break;
-      if (wide > 0 && cnt > wide && wide_levels-- == 0) return -1;
+      if (wide > 0 && cnt > wide && wide_levels-- == 0) return -1 - level;
       if (tid == 0) {
         S.cnt[(level + 2) % 3] = 0;
         // (filled in the level that uses it, and read after that level's barrier: the next level's
@@ -564,6 +566,8 @@ struct WgSolver {
       const int levels = relabel(round == 0 ? wide : 0, wide_levels, round > 0);
       if (levels < 0) {
         o.status = 3;
+        o.levels = -1 - levels;
+        o.t_relabel = (long long)wall_clock64() - t0;
         break;
       }
       o.levels += levels;

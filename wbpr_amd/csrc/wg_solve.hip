@@ -41,7 +41,7 @@ __device__ __forceinline__ void write_report(WgReport *rep, const WgOutcome &o, 
 }
 
 // A single graph.  Its heights and excesses go to global memory at the end, where the read-back
-// entry points expect them.
+// entry points, or a global relabel that goes on from an abandoned one, expect them.
 template <class L, int KIND>
 __global__ __launch_bounds__(kWgThreads) void k_wg_solve(L g, WgSingle a) {
   extern __shared__ __align__(16) char lds[];
@@ -50,13 +50,11 @@ __global__ __launch_bounds__(kWgThreads) void k_wg_solve(L g, WgSingle a) {
   w.st = WgStats{0, 0, 0, 0, 0, 0};
   w.carve(lds, a.lds_bytes, a.h, a.e);
   const WgOutcome o = w.solve(a.ratio, a.max_cycles, a.max_rounds, a.wide, a.wide_levels);
-  if (o.status != 3) {
-    for (int v = (int)threadIdx.x; v < a.n; v += kWgThreads) {
-      a.h[v] = w.h[v];
-      if constexpr (KIND == kWgBoth) a.e[v] = w.e[v];
-    }
-    if (threadIdx.x == 0) a.values[0] = o.value;
+  for (int v = (int)threadIdx.x; v < a.n; v += kWgThreads) {
+    a.h[v] = w.h[v];
+    if constexpr (KIND == kWgBoth) a.e[v] = w.e[v];
   }
+  if (threadIdx.x == 0) a.values[0] = o.value;
   write_report(a.report, o, w.st);
 }
 
