@@ -139,3 +139,23 @@ def test_grid_goes_on_from_an_abandoned_search(mf, orc, ctx, width, length, coop
         finally:
             dg.close()
     assert ctx.solve_noalloc(g, mf.ALGO_VC, bfs_cooperative=coop).value == value
+
+
+@pytest.mark.parametrize("left,right,both_lines", [
+    (9200, 9150, True), (9250, 9201, False),      # the sink takes less: frontiers up to 9,200 stay
+    (11400, 11800, True), (11400, 11801, False),  # more: up to 11,800
+])
+def test_wide_frontiers_by_layout(mf, orc, ctx, left, right, both_lines):
+    # matchings in one workgroup: any width on BCSR, what RCSR and BCSR2 read a slot's two lines for
+    g = mf.gen_bipartite(left, right, 8.0, seed=left)
+    value = orc.dinic_maxflow(g)
+    for layout in (mf.LAYOUT_BCSR, mf.LAYOUT_BCSR2, mf.LAYOUT_RCSR):
+        dg = ctx.upload(g, layout)
+        try:
+            r = dg.solve(mf.ALGO_VC)
+            assert r.value == value
+            assert (r.bfs_grid_levels == 0) == (layout == mf.LAYOUT_BCSR or both_lines)
+            assert orc.certify(g, dg.read_flow(return_excess=False), value,
+                               preflow=True)[0] == "ok"
+        finally:
+            dg.close()

@@ -9,6 +9,14 @@
 
 namespace mfk {
 enum WgKind { kWgBoth = 0, kWgHeights = 1, kWgGlobal = 2 };  // see wg_solve.h
+
+// When the first global relabel gives a solve up: once more than `levels` frontiers held more than
+// `from` vertices (0: never), or one more than `most` -- more than `most_short` where the sink takes
+// less than the source gives.
+struct WgWide {
+  int from, levels, most, most_short;
+};
+constexpr WgWide kWgNeverWide{0, 0, 0, 0};
 }
 
 namespace mf {
@@ -28,8 +36,7 @@ struct WgSingle {
   float ratio;         // cycle time / relabel time per round
   int max_cycles;      // cycles per round
   long long max_rounds;
-  int wide;            // > 0: give up when more than wide_levels frontiers of the first relabel
-  int wide_levels;     // hold more vertices than this
+  mfk::WgWide wide;
   long long *values;   // [0] receives the value
   WgReport *report;    // device memory
   int lds_bytes;       // (set by the launch)

@@ -61,6 +61,7 @@ struct WgShared {
   int nhub[3];  // hubs waiting, same rotation
   int chunk;    // items of the chunk list while an overflowed worklist is walked
   int flag;     // a source was reached
+  long long surplus;
   int stop[2];
   int hub[2][kWgHubCap];
 };
@@ -481,11 +482,35 @@ struct WgSolver {
     expand<B>(u, r, lane, T, level, check, out, ocnt);
   }
 
+  // Capacity out of the source less capacity into the sink.
+  __device__ __forceinline__ long long surplus() {
+    const int tid = (int)threadIdx.x;
+    if (tid == 0) S.surplus = 0;
+    __syncthreads();
+    long long sum = 0;
+    Range r = range(s);
+    for (int i = tid; i < r.d; i += BS) {
+      int w, res, key;
+      g.scan(r.seg(i), r.at(i), w, res, key);
+      if (w - vb != s) sum += res;
+    }
+    r = range(t);
+    for (int i = tid; i < r.d; i += BS) {
+      int w, idx;
+      g.bfs_slot(r.seg(i), r.at(i), w, idx);
+      if (w - vb != t) sum -= g.bfs_rin(r.seg(i), idx);
+    }
+    sum = tile_sum<64>(sum);
+    if (__lane_id() == 0)
+      atomicAdd(reinterpret_cast<unsigned long long *>(&S.surplus), (unsigned long long)sum);
+    __syncthreads();
+    return S.surplus;
+  }
+
   // Heights from a BFS over reverse residual arcs: distances to the sink, n where it cannot be
-  // reached.  Returns the levels; wide > 0 gives up once more than wide_levels frontiers held more
-  // vertices than that, before anything outside LDS has been written: -1 - level, the heights up to
-  // that level set.
-  __device__ __forceinline__ int relabel(int wide, int wide_levels, bool check) {
+  // reached.  Returns the levels; wide.from > 0 gives up (WgWide), before anything outside LDS has been
+  // written: -1 - level, the heights up to that level set.
+  __device__ __forceinline__ int relabel(const WgWide &wide, bool check) {
     const int tid = (int)threadIdx.x;
     for (int v = tid; v < n; v += BS) h[v] = (HT)(v == s ? n + 1 : (v == t ? 0 : n));
     for (int w = tid; w < wg_bits_words(n); w += BS) {
@@ -503,11 +528,12 @@ struct WgSolver {
       list(0)[0] = (HT)t;
     }
     __syncthreads();
-    int level = 0;
+    int level = 0, left = wide.levels, most = wide.most;
+    if (wide.from > 0 && wide.most_short < wide.most && surplus() > 0) most = wide.most_short;
     for (;; ++level) {
       const int cnt = S.cnt[level % 3];
       if (cnt == 0) break;
-      if (wide > 0 && cnt > wide && wide_levels-- == 0) return -1 - level;
+      if (wide.from > 0 && cnt > wide.from && (cnt > most || left-- == 0)) return -1 - level;
       if (tid == 0) {
         S.cnt[(level + 2) % 3] = 0;
         // (filled in the level that uses it, and read after that level's barrier: the next level's
@@ -546,7 +572,7 @@ struct WgSolver {
   // The residuals hold the capacities and every excess is zero on entry.  Every thread of the
   // workgroup calls this and returns the same outcome (source_out aside).
   __device__ __forceinline__ WgOutcome solve(float ratio, int max_cycles, long long max_rounds,
-                                             int wide, int wide_levels) {
+                                             const WgWide &wide) {
     const int tid = (int)threadIdx.x;
     WgOutcome o{0, 0, 0, 0, 0, 0, 0, 0};
     if constexpr (KIND == kWgBoth) {
@@ -563,7 +589,7 @@ struct WgSolver {
         break;
       }
       const long long t0 = (long long)wall_clock64();
-      const int levels = relabel(round == 0 ? wide : 0, wide_levels, round > 0);
+      const int levels = relabel(round == 0 ? wide : kWgNeverWide, round > 0);
       if (levels < 0) {
         o.status = 3;
         o.levels = -1 - levels;

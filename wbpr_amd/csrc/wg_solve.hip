@@ -49,7 +49,7 @@ __global__ __launch_bounds__(kWgThreads) void k_wg_solve(L g, WgSingle a) {
   WgSolver<L, KIND, kWgThreads> w{g, S, 0, a.n, a.s, a.t};
   w.st = WgStats{0, 0, 0, 0, 0, 0};
   w.carve(lds, a.lds_bytes, a.h, a.e);
-  const WgOutcome o = w.solve(a.ratio, a.max_cycles, a.max_rounds, a.wide, a.wide_levels);
+  const WgOutcome o = w.solve(a.ratio, a.max_cycles, a.max_rounds, a.wide);
   for (int v = (int)threadIdx.x; v < a.n; v += kWgThreads) {
     a.h[v] = w.h[v];
     if constexpr (KIND == kWgBoth) a.e[v] = w.e[v];
@@ -100,7 +100,7 @@ __device__ __forceinline__ void batch_one(const LayoutBCSR &g, const WgBatch &a,
   WgSolver<LayoutBCSR, KIND, BS> w{g, S, vb, a.nver[inst], a.src[inst] - vb, a.snk[inst] - vb};
   w.st = WgStats{0, 0, 0, 0, 0, 0};
   w.carve(lds, a.lds_bytes, a.h, a.e);
-  const WgOutcome o = w.solve(a.ratio, a.max_cycles, a.max_rounds, 0, 0);
+  const WgOutcome o = w.solve(a.ratio, a.max_cycles, a.max_rounds, kWgNeverWide);
   if (threadIdx.x == 0) {
     a.values[inst] = o.value;
     a.status[inst] = o.status;
