@@ -159,3 +159,33 @@ def test_wide_frontiers_by_layout(mf, orc, ctx, left, right, both_lines):
                                preflow=True)[0] == "ok"
         finally:
             dg.close()
+
+
+def test_graphs_destroyed_by_another_thread(mf, orc):
+    # a garbage collector's thread closes graphs of a context that is solving, launches being captured
+    import threading
+
+    ctx = mf.Context(0)
+    g = mf.gen_rmat(13, 8, seed=2)
+    value = orc.dinic_maxflow(g)
+    old = [ctx.upload(mf.gen_washington_rlg(8, 8, 100, i), mf.LAYOUT_BCSR) for i in range(400)]
+    done = threading.Event()
+
+    def collect():
+        while old and not done.is_set():
+            old.pop().close()
+            done.wait(0.0002)
+
+    thread = threading.Thread(target=collect)
+    thread.start()
+    try:
+        for cycles in range(6, 66, 6):
+            dg = ctx.upload(g, mf.LAYOUT_BCSR)
+            assert dg.solve(mf.ALGO_VC, cycle_graphs=1, cycles_per_relabel=cycles).value == value
+            dg.close()
+    finally:
+        done.set()
+        thread.join()
+        for dg in old:
+            dg.close()
+        ctx.close()

@@ -7,7 +7,7 @@
 // what is beyond the limit are given back at once, the rest with the context.  A context
 // belongs to one host thread at a time, and its calls end with their stream idle: a block on the
 // list has no work in flight.  The lock is for handles that another thread destroys (a garbage
-// collector's), as hipFree allowed.
+// collector's), as hipFree allowed, also while a call on other handles of the context runs.
 #pragma once
 
 #include <hip/hip_runtime.h>

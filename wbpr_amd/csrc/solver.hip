@@ -2773,8 +2773,15 @@ enum {
 // counter c of triple-buffer slot q of the frontier (CTL_FCNT) or worklist (CTL_CCNT) set
 constexpr int ctl_cnt(int set, int q, int c) { return set + (q * kNumClasses + c) * kCtlStride; }
 
+// Every call ends with its stream idle, after an error too: what it releases may be used again at once.
+static mf_status drained(mf_context *ctx, mf_status st) {
+  if (st != MF_OK) (void)hipStreamSynchronize(ctx->stream);
+  return st;
+}
+
+// (Waits for nothing: no call on the graph is running, and another thread may be, on other graphs of
+// the context -- a wait would break its capture.)
 static void free_dev(mf_context *ctx, DevGraph *g) {
-  (void)hipStreamSynchronize(ctx->stream);  // (after an error)
   for (auto &cg : g->cycle_graphs)
     for (hipGraphExec_t x : cg.exec)
       if (x) (void)hipGraphExecDestroy(x);
@@ -2900,8 +2907,9 @@ static mf_status set_vertex_classes(mf_context *ctx, DevGraph &G,
 // matchings of 256 to 65,536 vertices a side: the tables were 300 of a call's 720 ms, on the host.)
 enum class Keep { kAll, kBatchTables, kBatch, kBatchOnce };
 
-static mf_status upload(mf_context *ctx, const mf_csr *c, const int32_t *src, const int32_t *snk,
-                        int32_t k, mf_layout layout, DevGraph &G, Keep keep = Keep::kAll) {
+static mf_status upload_now(mf_context *ctx, const mf_csr *c, const int32_t *src,
+                            const int32_t *snk, int32_t k, mf_layout layout, DevGraph &G,
+                            Keep keep) {
   const bool keep_host = keep == Keep::kAll;
   const bool tables = keep == Keep::kAll || keep == Keep::kBatchTables;
   G.owner = ctx;
@@ -3045,6 +3053,11 @@ static mf_status upload(mf_context *ctx, const mf_csr *c, const int32_t *src, co
   HIP_TRY(hipStreamSynchronize(st));
   G.fresh = true;  // the layout build wrote every residual as its capacity
   return MF_OK;
+}
+
+static mf_status upload(mf_context *ctx, const mf_csr *c, const int32_t *src, const int32_t *snk,
+                        int32_t k, mf_layout layout, DevGraph &G, Keep keep = Keep::kAll) {
+  return drained(ctx, upload_now(ctx, c, src, snk, k, layout, G, keep));
 }
 
 // Residuals back to the capacities, unless no solve has run since the layout was built.
@@ -3757,9 +3770,9 @@ static mf_status run_solve(mf_context *ctx, DevGraph &G, const L &lay, mf_algo a
 
 mf_status solve_graph(mf_context *ctx, DevGraph &G, mf_algo algo, const mf_options &o,
                       mf_result *res) {
-  if (G.layout == MF_LAYOUT_BCSR) return run_solve(ctx, G, G.bcsr(), algo, o, res);
-  if (G.layout == MF_LAYOUT_BCSR2) return run_solve(ctx, G, G.bcsr2(), algo, o, res);
-  return run_solve(ctx, G, G.rcsr(), algo, o, res);
+  return drained(ctx, G.layout == MF_LAYOUT_BCSR    ? run_solve(ctx, G, G.bcsr(), algo, o, res)
+                      : G.layout == MF_LAYOUT_BCSR2 ? run_solve(ctx, G, G.bcsr2(), algo, o, res)
+                                                    : run_solve(ctx, G, G.rcsr(), algo, o, res));
 }
 
 static mf_status check_options(const mf_options &o) {
@@ -4809,6 +4822,7 @@ mf_status mf_rcsr_push_relabel(mf_context *ctx, int algo_type, int V, int E, int
   for (int32_t i = cpu_offsets[source]; i < cpu_offsets[source + 1]; ++i)
     if (cpu_destinations[i] != source) sc += cpu_capacities[i];
   auto fail = [&](mf_status code) {
+    (void)drained(ctx, code);
     free_dev(ctx, &G);
     return code;
   };
