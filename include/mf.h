@@ -330,7 +330,8 @@ mf_status mf_batch_autotune(mf_context *ctx, const mf_csr *inst, int32_t k, int3
  * ranges are reused when it finishes.  A larger request runs alone on the whole grid from one of
  * max_inflight_launches worker contexts (each with its own stream), with device memory charged
  * to the other half of the budget (mf_footprint_bytes); those solves overlap on the device with
- * the serving kernel.  Admission goes through pending requests in arrival order and admits each
+ * the serving kernel.  What the requests in flight leave of that half, the worker contexts may hold
+ * as freed blocks for the next requests.  Admission goes through pending requests in arrival order and admits each
  * one that fits now.  Every call takes the server's lock, so calls may come from several
  * threads. */
 typedef struct mf_server mf_server;

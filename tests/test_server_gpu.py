@@ -79,3 +79,8 @@ def test_power_law_requests(mf, orc, ctx, scale, factor):
         assert min(srv.times(i)["device_ms"] for i in ids) < 20
     finally:
         srv.close()
+
+
+def test_large_request_frees_nothing_beside_a_backlog(mf, orc, ctx):
+    # hipFree waits for the serving kernel: the arrays of a request of 70 MB are kept for the next one
+    assert max(beside_backlog(mf, orc, ctx, mf.gen_rmat(16, 16, seed=4))) >= 256

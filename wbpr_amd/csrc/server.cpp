@@ -10,7 +10,8 @@
 //   - alone (larger requests): one workgroup would take tens of milliseconds on them, so each
 //     runs on the whole grid (the single-instance solver) from a worker thread with its own
 //     context and stream, overlapping on the device with the serving kernel and other large
-//     requests.  Its device memory is allocated per request and charged to the budget.
+//     requests.  Its device memory is charged to the budget, and kept for the next request as far as
+//     the requests in flight leave room.
 // The budget (hbm_budget_bytes) is split: half for the arena, half for the large requests in
 // flight.  Admission goes through the pending requests in arrival order and admits every one
 // that fits now, so a request waiting for memory does not hold up smaller ones behind it.
@@ -151,7 +152,7 @@ struct mf_server {
   double first_submit = -1, last_finish = 0;
   int64_t next_id = 1;
   mf_server_stats st{};
-  std::mutex mu;
+  std::mutex mu, share_mu;  // share_mu before mu
   std::condition_variable cv;
 };
 
@@ -200,7 +201,20 @@ static void reverse_if_cheaper(Request &r) {
   for (int32_t &c : r.cap) c = ~c;
 }
 
+// Worker contexts keep freed blocks for the next request (a hipFree waits for the serving kernel) in what
+// the requests in flight leave of their half of the budget.  Called before a request allocates.
+static void share_alone_budget(mf_server *srv) {
+  std::lock_guard<std::mutex> share(srv->share_mu);  // the last to set the limits saw all in flight
+  int64_t left;
+  {
+    std::lock_guard<std::mutex> lk(srv->mu);
+    left = srv->alone_budget - srv->alone_in_use;
+  }
+  for (mf_context *c : srv->ctxs) context_pool_limit(c, (size_t)(left / (int64_t)srv->ctxs.size()));
+}
+
 static void run_alone(mf_server *srv, Launch *L) {
+  share_alone_budget(srv);
   Request &r = *L->req;
   const mf_csr c = r.view();
   mf_options o;
@@ -417,8 +431,6 @@ mf_status mf_server_create(mf_context *ctx, int64_t hbm_budget_bytes, int32_t ma
       serve_arena_destroy(srv->arena);
       return s;
     }
-    // what the worker contexts keep between requests: an eighth of their half of the budget
-    context_pool_limit(c, (size_t)(srv->alone_budget / (8 * max_inflight_launches)));
     srv->ctxs.push_back(c);
     srv->ctx_busy.push_back(false);
   }

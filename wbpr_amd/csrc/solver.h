@@ -111,7 +111,7 @@ bool serve_running(ServeArena *a);
 mf_status serve_launch(ServeArena *a);
 // The device a context runs on.
 int context_device(const mf_context *ctx);
-// Bytes of freed device memory the context may keep for its next call (DevPool).
+// Bytes of device memory the context may hold beyond what its calls need (DevPool).  From any thread.
 void context_pool_limit(mf_context *ctx, size_t bytes);
 int64_t serve_launches(const ServeArena *a);
 }  // namespace mf

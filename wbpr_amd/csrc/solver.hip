@@ -4277,7 +4277,7 @@ int64_t serve_launches(const ServeArena *a) { return a->launches; }
 
 int context_device(const mf_context *ctx) { return ctx->device; }
 
-void context_pool_limit(mf_context *ctx, size_t bytes) { ctx->pool.limit = bytes; }
+void context_pool_limit(mf_context *ctx, size_t bytes) { ctx->pool.set_limit(bytes, bytes); }
 
 void *context_staging(mf_context *ctx, size_t bytes) {
   if (ctx->staging_bytes >= bytes) return ctx->staging;
