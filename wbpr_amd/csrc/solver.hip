@@ -4065,13 +4065,15 @@ void batch_release(BatchResident *r) {
 // to 156 KB, k_bfs_wg has 56 KB): the serving grid leaves CUs free for those (serve_groups).
 constexpr int kServeLds = 112 << 10;
 static_assert(wg_kind(kServeVertices, kServeLds) == kWgBoth, "every served instance fits");
-constexpr int kXcds = 8;
-// Workgroups of the serving kernel: one to a CU, but for as many CUs of every XCD as solves may run
-// alone at a time.  A solve has one such kernel in flight, and the only workgroup of a launch always
-// goes to the first XCD, as workgroup i does to XCD i mod 8.  (With a workgroup on every CU a request
-// of 18,000 vertices waited for 42 to 64 ms beside 600 of 13 to 22 ms, whatever the queue held last.)
+constexpr int kEngines = 32;  // shader engines: four to each of the eight XCDs
+// Workgroups of the serving kernel: one to a CU, but for one CU of every shader engine for up to four
+// solves that may run alone at a time.  Such a solve has one large workgroup in flight, and a
+// workgroup waits for the engine whose turn it is, whatever the others have free: with a CU of
+// every XCD left to one solve at a time, half of the servers tried still held it up.  (With a
+// workgroup on every CU a request of 18,000 vertices waited for 42 to 64 ms beside 600 of 13 to 22 ms,
+// whatever the queue held last.)
 static int serve_groups(int num_cu, int alone) {
-  return std::max(num_cu / 2, num_cu - kXcds * alone);
+  return std::max(num_cu / 2, num_cu - kEngines * ((alone + 3) / 4));
 }
 constexpr long long kServeIdleTicks = 200000;      // 2 ms at the 100 MHz wall clock
 
