@@ -94,3 +94,32 @@ def test_one_large_request_at_a_time_beside_a_backlog(mf, orc, ctx):
     for c in others:
         c.close()
     assert sorted(behind)[1] >= 256, behind  # (one server's streams may share a hardware queue)
+
+
+@pytest.mark.parametrize("others", [0, 1, 2])
+@pytest.mark.parametrize("alone_at_a_time", [1, 4])
+def test_no_stream_waits_for_the_serving_kernel(mf, orc, ctx, others, alone_at_a_time):
+    # whatever streams there were before the server's: none of a large request's work shares a hardware
+    # queue with the serving kernel
+    others = [mf.Context(0) for _ in range(others)]
+    big = mf.gen_bipartite(20000, 15000, 8.0, 77)
+    behind = beside_backlog(mf, orc, ctx, big, alone_at_a_time=alone_at_a_time)
+    for c in others:
+        c.close()
+    assert min(behind) >= 256, behind
+
+
+def test_small_requests_behind_large_ones(mf, orc, ctx):
+    # eight large requests, one of them perhaps in the serving kernel's hardware queue, then small ones:
+    # the serving kernel is launched when that one has finished
+    large = [mf.gen_genrmf(18, 56, 1, 10000, i) for i in range(8)]
+    small = [mf.gen_washington_rlg(20 + i, 30, 10000, i) for i in range(24)]
+    srv = mf.Server(ctx, hbm_budget_bytes=4 << 30, max_inflight_launches=4)
+    try:
+        for _ in range(3):
+            ids = [srv.submit(g) for g in large]
+            srv.progress()
+            ids += [srv.submit(g) for g in small]
+            assert serve(srv, ids) == [orc.dinic_maxflow(g) for g in large + small]
+    finally:
+        srv.close()

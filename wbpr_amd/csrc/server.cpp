@@ -41,6 +41,11 @@ constexpr int64_t kSoloArcs = 262144;
 constexpr int32_t kQueueCap = 4096;    // entries of the serving kernel's queue ring
 constexpr int64_t kSlotsPerVertex = 10;  // arena slot capacity per vertex (S = 2m ~ 10n typical)
 
+// Worker contexts whose streams are kept out of the serving kernel's hardware queue: HIP makes four
+// queues.  The others take what they get, for the fourth queue is worth having while the serving
+// kernel does not run (128 requests, 34 of them alone: 165 ms with it, 208 without).
+constexpr int32_t kApartContexts = 3;
+
 enum State { PENDING = 0, COPYING, PUBLISHED, RUNNING_ALONE, DONE, FAILED };
 
 double now_ms() {
@@ -143,6 +148,7 @@ struct mf_server {
   // alone path
   std::vector<mf_context *> ctxs;
   std::vector<bool> ctx_busy;
+  std::vector<bool> ctx_apart;  // the context's stream shares no hardware queue with the serving kernel
   std::vector<std::unique_ptr<Launch>> inflight;
   // all requests
   std::deque<std::shared_ptr<Request>> pending;
@@ -311,6 +317,28 @@ static void publish_copied(mf_server *srv) {
   }
 }
 
+// A worker context for a request that runs alone, or -1 (lock held).  What shares the serving kernel's
+// hardware queue takes one only while there is nothing to serve, and that kernel is not launched
+// before it has finished (step): neither waits for the other for longer than one solve.
+static int free_context(mf_server *srv) {
+  int shared = -1;
+  for (size_t c = 0; c < srv->ctx_busy.size(); ++c) {
+    if (srv->ctx_busy[c]) continue;
+    if (srv->ctx_apart[c]) return (int)c;
+    shared = (int)c;
+  }
+  if (shared < 0 || !srv->copying.empty() || !srv->published.empty()) return -1;
+  for (const auto &r : srv->pending)
+    if (r->batched) return -1;
+  return serve_running(srv->arena) ? -1 : shared;
+}
+
+static bool queue_shared(const mf_server *srv) {
+  for (size_t c = 0; c < srv->ctx_busy.size(); ++c)
+    if (srv->ctx_busy[c] && !srv->ctx_apart[c]) return true;
+  return false;
+}
+
 // Admits pending requests in arrival order, every one that fits now (lock held).
 static void admit(mf_server *srv) {
   for (size_t i = 0; i < srv->pending.size();) {
@@ -340,12 +368,7 @@ static void admit(mf_server *srv) {
         }
       }
     } else if (srv->alone_in_use + r.footprint <= srv->alone_budget) {
-      int slot = -1;
-      for (size_t c = 0; c < srv->ctx_busy.size(); ++c)
-        if (!srv->ctx_busy[c]) {
-          slot = (int)c;
-          break;
-        }
+      const int slot = free_context(srv);
       if (slot >= 0) {
         srv->alone_in_use += r.footprint;
         srv->ctx_busy[(size_t)slot] = true;
@@ -383,7 +406,7 @@ static mf_status step(mf_server *srv, std::unique_lock<std::mutex> &lk) {
   // was solved while this step admitted or copied is not mistaken for one left unclaimed
   const bool running = serve_running(srv->arena);
   if (!running) poll_batched(srv);
-  if (!srv->published.empty() && !running) {
+  if (!srv->published.empty() && !running && !queue_shared(srv)) {
     const mf_status s = serve_launch(srv->arena);
     if (s != MF_OK) return s;
     srv->st.launches++;
@@ -432,6 +455,7 @@ mf_status mf_server_create(mf_context *ctx, int64_t hbm_budget_bytes, int32_t ma
       return s;
     }
     srv->ctxs.push_back(c);
+    srv->ctx_apart.push_back(serve_stream_apart(srv->arena, c, i < kApartContexts));
     srv->ctx_busy.push_back(false);
   }
   *out = srv.release();

@@ -93,6 +93,9 @@ int64_t serve_arena_bytes(int64_t nv, int64_t ns);
 // alone: solves that may run beside the serving kernel at a time, which leaves CUs for them.
 mf_status serve_arena_create(mf_context *ctx, int64_t nv, int64_t ns, int32_t qcap, int32_t alone,
                              ServeArena **out);
+// Whether the stream of an idle context shares no hardware queue with the serving kernel; find: after
+// replacing it by one that does not, if there is one.
+bool serve_stream_apart(ServeArena *a, mf_context *ctx, bool find);
 // Leaves idle workgroups, waits for the kernel and the copies, frees everything.
 void serve_arena_destroy(ServeArena *a);
 // Queues the copies of inst into vertices [vb, vb + n] and slots [sb, sb + S) of the arena;

@@ -2516,6 +2516,18 @@ __global__ __launch_bounds__(kBlock) void k_serve_wg(L g, ServeArgs a) {
   block_flush(nv, ns, 0, 0, a.b.stats, ST_BFS_VERTS);
 }
 
+// Holds its stream until *release is set, for `ticks` of the wall clock at most (see apart).
+__global__ void k_hold(const int *release, long long ticks) {
+  const long long t0 = (long long)wall_clock64();
+  while ((long long)wall_clock64() - t0 < ticks &&
+         !__hip_atomic_load(release, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM))
+    __builtin_amdgcn_s_sleep(32);
+}
+
+__global__ void k_mark(int *word) {
+  __hip_atomic_store(word, 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 }  // namespace mf
 
 // ============================================================================================
@@ -4093,7 +4105,7 @@ struct ServeArena {
   // host memory the GPU reads and writes uncached
   int *entries = nullptr;
   ServeReport *reports = nullptr;
-  int *pub = nullptr;  // [0] published count, [1] closed
+  int *pub = nullptr;  // [0] published count, [1] closed, [2..3] words of apart()
   hipStream_t copy_stream = nullptr, kernel_stream = nullptr;
   bool launched = false;
   int64_t launches = 0;
@@ -4114,6 +4126,49 @@ void serve_arena_destroy(ServeArena *a) {
   if (a->copy_stream) (void)hipStreamDestroy(a->copy_stream);
   if (a->kernel_stream) (void)hipStreamDestroy(a->kernel_stream);
   delete a;
+}
+
+// Streams share a few hardware queues, and a kernel waits for the ones before it in its queue, whatever
+// their streams: work in the serving kernel's queue waits until that kernel leaves, without bound
+// under a lasting backlog.  HIP does not say which streams share one, so it is tried out when a server
+// is created: whether a kernel on st runs while one on `held` does.
+constexpr long long kHoldTicks = 2000000;  // 20 ms, ended by the host after kHoldMs at most
+constexpr double kHoldMs = 0.3;            // a kernel that is not behind `held` starts within 0.05 ms
+constexpr int kQueueTries = 8;             // (HIP makes four queues unless told otherwise)
+
+static bool apart(ServeArena *a, hipStream_t held, hipStream_t st) {
+  int *words = nullptr;
+  if (hipHostGetDevicePointer((void **)&words, a->pub, 0) != hipSuccess) return true;
+  __atomic_store_n(&a->pub[2], 0, __ATOMIC_RELAXED);
+  __atomic_store_n(&a->pub[3], 0, __ATOMIC_RELEASE);
+  k_hold<<<1, 1, 0, held>>>(words + 2, kHoldTicks);
+  k_mark<<<1, 1, 0, st>>>(words + 3);
+  const double t0 = now_ms();
+  bool ran = false;
+  while (!ran && now_ms() - t0 < kHoldMs) ran = __atomic_load_n(&a->pub[3], __ATOMIC_ACQUIRE) != 0;
+  __atomic_store_n(&a->pub[2], 1, __ATOMIC_RELEASE);
+  (void)hipStreamSynchronize(held);
+  (void)hipStreamSynchronize(st);
+  return ran;
+}
+
+// Replaces *st by new streams until ok() holds, kQueueTries times at most.
+template <class Ok>
+static void find_stream(hipStream_t *st, Ok ok) {
+  std::vector<hipStream_t> others;
+  hipStream_t next = nullptr;
+  for (int q = 0; q < kQueueTries && !ok(); ++q) {
+    if (hipStreamCreateWithFlags(&next, hipStreamNonBlocking) != hipSuccess) break;
+    others.push_back(*st);
+    *st = next;
+  }
+  for (hipStream_t x : others) (void)hipStreamDestroy(x);
+}
+
+bool serve_stream_apart(ServeArena *a, mf_context *ctx, bool find) {
+  auto ok = [&] { return apart(a, a->kernel_stream, ctx->stream); };
+  if (find) find_stream(&ctx->stream, ok);
+  return ok();
 }
 
 int64_t serve_arena_bytes(int64_t nv, int64_t ns) {
@@ -4167,6 +4222,11 @@ mf_status serve_arena_create(mf_context *ctx, int64_t nv, int64_t ns, int32_t qc
                      a->kernel_stream) != hipSuccess ||
       hipStreamSynchronize(a->kernel_stream) != hipSuccess)
     return fail(MF_ERR_DEVICE);
+  (void)apart(a, a->kernel_stream, a->copy_stream);  // (the first launch takes longer)
+  find_stream(&a->kernel_stream, [&] {  // (the null stream: synchronous copies)
+    return apart(a, a->kernel_stream, a->copy_stream) && apart(a, a->kernel_stream, nullptr) &&
+           apart(a, a->kernel_stream, ctx->stream);
+  });
   *out = a;
   return MF_OK;
 }
