@@ -114,12 +114,13 @@ def test_small_requests_behind_large_ones(mf, orc, ctx):
     # the serving kernel is launched when that one has finished
     large = [mf.gen_genrmf(18, 56, 1, 10000, i) for i in range(8)]
     small = [mf.gen_washington_rlg(20 + i, 30, 10000, i) for i in range(24)]
+    values = [orc.dinic_maxflow(g) for g in large + small]
     srv = mf.Server(ctx, hbm_budget_bytes=4 << 30, max_inflight_launches=4)
     try:
         for _ in range(3):
             ids = [srv.submit(g) for g in large]
             srv.progress()
             ids += [srv.submit(g) for g in small]
-            assert serve(srv, ids) == [orc.dinic_maxflow(g) for g in large + small]
+            assert serve(srv, ids) == values
     finally:
         srv.close()
