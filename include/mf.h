@@ -82,6 +82,13 @@ typedef struct mf_host_graph {
   int64_t m_processed;      /* arc lines read (CSRGraph::num_edges_processed) */
 } mf_host_graph;
 
+/* Graphs whose heights fit one CU's LDS (up to about 63,000 vertices; with more than 65,536 residual
+ * slots only graphs of low degree with narrow frontiers) are solved inside one workgroup, and so is
+ * every instance of a batch (batch_mode 0) of up to 2^19 vertices.  TC and VC are the same there, and
+ * tile_lanes, class_lanes, forward_hops, bfs_block_frontier, bfs_cooperative and batch_algo have no
+ * effect.  verbose, profile_kernels, record_workload, cycle_graphs and bfs_direction 1 and 2 belong to
+ * the grid-wide kernels and keep a single graph on them: what they report is not the one-workgroup
+ * solve (a 64 x 64 random level graph takes 10.7 ms with profile_kernels, 2.2 without). */
 typedef struct mf_options {
   int32_t cycles_per_relabel; /* fixed push-relabel cycles between global relabels; 0 = adaptive */
   int32_t tile_lanes;         /* VC lanes per vertex: 0 = by degree bucket, else 1/8/16/32/64/256 */
@@ -94,7 +101,8 @@ typedef struct mf_options {
                                  (its variant for graphs of low degree: eight times this) */
   float relabel_time_ratio;   /* adaptive cadence: after a global relabel taking T ms, cycles run
                                  for about ratio * T ms; 0 = default (2) */
-  int32_t batch_algo;         /* mf_batch_solve: 0 = TC (default), 1 = VC */
+  int32_t batch_algo;         /* mf_batch_solve, batch_mode 1 and instances of more than 2^19 vertices:
+                                 0 = TC (default), 1 = VC */
   int32_t batch_mode;         /* mf_batch_solve: 0 = one workgroup per instance (default),
                                  1 = all instances as one packed graph on the whole grid */
   int32_t bfs_direction;      /* global relabel: 0 = bottom-up levels while the frontier is large
@@ -274,7 +282,8 @@ mf_status mf_solve_noalloc(mf_context *ctx, const mf_csr *g, mf_algo algo, mf_la
  * widths (class_lanes, VC only), relabel cadences (relabel_time_ratio, or a fixed
  * cycles_per_relabel scaled from the cycles per round the starting options ran), forwarding
  * (forward_hops), graph replay (cycle_graphs) and one-workgroup BFS
- * limits (bfs_block_frontier), starting from *base (NULL = defaults), by coordinate descent over
+ * limits (bfs_block_frontier), leaving out what has no effect on the graph (see mf_options), starting
+ * from *base (NULL = defaults), by coordinate descent over
  * the mean of three solves per candidate (the current best's estimate is the mean of all its
  * solves, re-timed before each sweep), with at least two sweeps over all parameters and a third
  * if the second changed one; the winner is then timed against the starting options (six solves
@@ -310,12 +319,14 @@ mf_status mf_rcsr_push_relabel(mf_context *ctx, int algo_type, int V, int E, int
  * offsets.  opts->batch_mode 0 (default): a persistent kernel whose workgroups pull whole
  * instances from a device queue, largest first, and solve each inside the workgroup;
  * batch_mode 1: the grid-wide kernels run over all instances at once.  opts->batch_algo picks
- * TC (0, default) or VC (1) cycles.  values[k] receives each value. */
+ * TC (0, default) or VC (1) cycles in batch_mode 1 and for instances of more than 2^19 vertices; the
+ * others are solved with their vertex state in LDS (see mf_options).  values[k] receives each value. */
 mf_status mf_batch_solve(mf_context *ctx, const mf_csr *inst, int32_t k, const mf_options *opts,
                          int64_t *values, mf_result *total);
 /* Autotuner of the batched solve: trial batched solves of a sample of at most `sample` instances
  * (the largest ones, which set the tail of a persistent launch, and an even spread of the rest)
- * over batch_algo and relabel_time_ratio; *best receives the fastest options. */
+ * over relabel_time_ratio and, where they have an effect (see mf_options), batch_algo, class_lanes and
+ * forward_hops; *best receives the fastest options. */
 mf_status mf_batch_autotune(mf_context *ctx, const mf_csr *inst, int32_t k, int32_t sample,
                             const mf_options *base, mf_options *best, double *best_ms,
                             int32_t *trials);
@@ -327,7 +338,7 @@ mf_status mf_batch_autotune(mf_context *ctx, const mf_csr *inst, int32_t k, int3
  * most 16,384 vertices and 262,144 arcs is laid out on the host at submit, admitted as soon as
  * arena ranges and a queue entry are free, copied into its ranges and published into the
  * running kernel's queue, where the next free workgroup solves it inside the running batch; its
- * ranges are reused when it finishes.  A larger request runs alone on the whole grid from one of
+ * ranges are reused when it finishes.  A larger request runs alone, as a single solve, from one of
  * max_inflight_launches worker contexts (each with its own stream), with device memory charged
  * to the other half of the budget (mf_footprint_bytes); those solves overlap on the device with
  * the serving kernel.  What the requests in flight leave of that half, the worker contexts may hold
@@ -350,7 +361,7 @@ typedef struct mf_server_times {
   double start_ms;    /* published into the running batch, or its launch started */
   double finish_ms;   /* the server saw its result */
   double device_ms;   /* the request's own solve on the device */
-  int32_t batched;    /* 1: solved inside the running batch; 0: alone on the whole grid */
+  int32_t batched;    /* 1: solved inside the running batch; 0: alone */
   int32_t reserved;
 } mf_server_times;
 mf_status mf_server_create(mf_context *ctx, int64_t hbm_budget_bytes, int32_t max_inflight_launches,

@@ -97,3 +97,20 @@ def test_hubs_with_excesses_in_global_memory(mf, orc, ctx, width, length, slots)
                                    preflow=True)[0] == "ok"
         finally:
             dg.close()
+
+
+def test_autotune_leaves_out_what_has_no_effect(mf, orc, ctx):
+    inert = ("tile_lanes", "class_lanes", "forward_hops", "batch_algo", "bfs_block_frontier",
+             "bfs_cooperative")
+    start = mf.options(class_lanes=[4, 8, 16, 64, 256], forward_hops=8,
+                       bfs_block_frontier=1024).to_dict()
+    g = chains(mf, 40, 60, seed=2)
+    best, _, trials = ctx.batch_autotune([g] * 8 + [chains(mf, 20, 30, seed=3)] * 8, sample=8, **start)
+    assert {k: best[k] for k in inert} == {k: start[k] for k in inert} and trials >= 18
+    dg = ctx.upload(g, mf.LAYOUT_BCSR)
+    try:
+        best, _, trials = dg.autotune(mf.ALGO_VC, **start)
+        assert best["cycle_graphs"] or {k: best[k] for k in inert} == {k: start[k] for k in inert}
+        assert dg.solve(mf.ALGO_VC, **best).value == orc.dinic_maxflow(g)
+    finally:
+        dg.close()

@@ -23,6 +23,9 @@
 //                     captured hipGraphs, cached on the resident graph, or launched one by one.
 //   batch algorithm   mf_options.batch_algo (batched solves only): TC or VC cycles.
 //
+// What has no effect is not tried: while the current best's solves run inside one workgroup, tile widths,
+// forwarding, BFS hand-over and the batch algorithm.
+//
 // Lock-free schedules differ from run to run (solve times spread by +-15% on long-path graphs),
 // so a candidate's time is the mean of three solves, the starting options' the mean of six, and
 // the current best's the mean of all its solves (it is timed again before every further sweep,
@@ -77,19 +80,21 @@ bool same_lanes(const uint16_t *a, const uint16_t *b) {
 }
 
 // One sweep over every parameter: each candidate value is tried with the others as they stand
-// in cur, which consider(t) replaces by t when t is faster (cur is the caller's live value).
+// in cur, which consider(t) replaces by t when t is faster (cur is the caller's live value, lds whether
+// its solves run inside one workgroup).
 // cadence_base: cycles per global-relabel round measured with the starting options (0: none).
 template <class Consider>
-mf_status sweep(const mf_options &cur, bool tune_lanes, bool tune_batch_algo,
+mf_status sweep(const mf_options &cur, const bool &lds, bool tune_lanes, bool tune_batch_algo,
                 double cadence_base, Consider consider) {
   mf_status st = MF_OK;
-  if (tune_batch_algo) {
+  if (tune_batch_algo && !lds) {
     mf_options t = cur;
     t.batch_algo = cur.batch_algo == 0 ? 1 : 0;
     if ((st = consider(t)) != MF_OK) return st;
   }
   if (tune_lanes && (!tune_batch_algo || cur.batch_algo == 1)) {
     for (const auto &p : kLanePresets) {
+      if (lds) break;
       if (same_lanes(p, cur.class_lanes)) continue;
       mf_options t = cur;
       std::memcpy(t.class_lanes, p, sizeof(t.class_lanes));
@@ -103,6 +108,7 @@ mf_status sweep(const mf_options &cur, bool tune_lanes, bool tune_batch_algo,
   }
   const int32_t h0 = cur.forward_hops;
   for (int32_t h : kForwardHops) {
+    if (lds) break;
     if (h == h0) continue;
     mf_options t = cur;
     t.forward_hops = h;
@@ -132,12 +138,13 @@ mf_status sweep(const mf_options &cur, bool tune_lanes, bool tune_batch_algo,
       if ((st = consider(t)) != MF_OK) return st;
     }
   }
-  if (!tune_batch_algo) {  // the batched kernel runs its BFS inside each workgroup anyway
+  if (!tune_batch_algo && !lds) {  // batched, the BFS runs inside each workgroup anyway
     mf_options c = cur;
     c.bfs_cooperative = cur.bfs_cooperative ? 0 : 1;
     if ((st = consider(c)) != MF_OK) return st;
     const int32_t f0 = effective_frontier(cur);
     for (int32_t f : kFrontiers) {
+      if (lds) break;
       if (f == f0) continue;
       mf_options t = cur;
       t.bfs_block_frontier = f;
@@ -147,8 +154,9 @@ mf_status sweep(const mf_options &cur, bool tune_lanes, bool tune_batch_algo,
   return MF_OK;
 }
 
-// Coordinate descent over the candidates; run(opts, ms, reps, cpr) times reps solves (mean ms)
-// and, when cpr is not null, stores their mean cycles per global-relabel round there.
+// Coordinate descent over the candidates; run(opts, ms, reps, cpr, lds) times reps solves (mean ms),
+// stores whether they ran inside one workgroup and, when cpr is not null, their mean cycles per
+// global-relabel round.
 template <class Run>
 mf_status descend(mf_options cur, bool tune_lanes, bool tune_batch_algo, Run run,
                   mf_options *best, double *best_ms) {
@@ -164,9 +172,10 @@ mf_status descend(mf_options cur, bool tune_lanes, bool tune_batch_algo, Run run
   // faster candidate can still replace them
   double cur_ms = 0, cur_sum = 0;
   int cur_n = 0;
+  bool lds = false;
   auto time_cur = [&](int reps, double *cpr) -> mf_status {
     double ms = 0;
-    const mf_status s = run(cur, ms, reps, cpr);
+    const mf_status s = run(cur, ms, reps, cpr, lds);
     if (s != MF_OK) return s;
     cur_sum += ms * reps;
     cur_n += reps;
@@ -180,10 +189,12 @@ mf_status descend(mf_options cur, bool tune_lanes, bool tune_batch_algo, Run run
   bool changed = false;
   auto consider = [&](const mf_options &t) -> mf_status {
     double ms = 0;
-    const mf_status s = run(t, ms, kRepeats, nullptr);
+    bool t_lds = false;
+    const mf_status s = run(t, ms, kRepeats, nullptr, t_lds);
     if (s != MF_OK) return s;
     if (ms < cur_ms) {
       cur = t;
+      lds = t_lds;
       cur_sum = ms * kRepeats;
       cur_n = kRepeats;
       cur_ms = ms;
@@ -195,7 +206,7 @@ mf_status descend(mf_options cur, bool tune_lanes, bool tune_batch_algo, Run run
     changed = false;
     if (pass > 0 && (st = time_cur(kRepeats, nullptr)) != MF_OK) return st;
     // sweep() reads cur live: each parameter is tried on top of the values chosen before it
-    if ((st = sweep(cur, tune_lanes, tune_batch_algo, cadence_base, consider)) != MF_OK)
+    if ((st = sweep(cur, lds, tune_lanes, tune_batch_algo, cadence_base, consider)) != MF_OK)
       return st;
     if (!changed && pass > 0) break;  // a second sweep always runs, against a re-timed best
   }
@@ -203,7 +214,9 @@ mf_status descend(mf_options cur, bool tune_lanes, bool tune_batch_algo, Run run
     double a_ms = 0, b_ms = 0;
     for (int r = 0; r < kValidate; ++r) {
       double x = 0, y = 0;
-      if ((st = run(start, x, 1, nullptr)) != MF_OK || (st = run(cur, y, 1, nullptr)) != MF_OK)
+      bool any = false;
+      if ((st = run(start, x, 1, nullptr, any)) != MF_OK ||
+          (st = run(cur, y, 1, nullptr, any)) != MF_OK)
         return st;
       a_ms += x / kValidate;
       b_ms += y / kValidate;
@@ -234,7 +247,7 @@ mf_status mf_autotune(mf_context *ctx, mf_graph *g, mf_algo algo, const mf_optio
   o.profile_kernels = 0;
   int64_t value = -1;
   int32_t n = 0;
-  auto run = [&](const mf_options &t, double &ms, int reps, double *cpr) -> mf_status {
+  auto run = [&](const mf_options &t, double &ms, int reps, double *cpr, bool &lds) -> mf_status {
     ms = 0;
     double cycles = 0, rounds = 0;
     for (int r = 0; r < reps; ++r) {
@@ -249,6 +262,7 @@ mf_status mf_autotune(mf_context *ctx, mf_graph *g, mf_algo algo, const mf_optio
       ++n;
     }
     if (cpr) *cpr = rounds > 0 ? cycles / rounds : 0;
+    lds = mf::graph_in_lds(g);
     return MF_OK;
   };
   const mf_status st =
@@ -296,7 +310,7 @@ mf_status mf_batch_autotune(mf_context *ctx, const mf_csr *inst, int32_t k, int3
   } release{resident};
   std::vector<int64_t> ref, vals(sub.size());
   int32_t n = 0;
-  auto run = [&](const mf_options &t, double &ms, int reps, double *cpr) -> mf_status {
+  auto run = [&](const mf_options &t, double &ms, int reps, double *cpr, bool &lds) -> mf_status {
     ms = 0;
     if (cpr) *cpr = 0;  // the batched kernel keeps its own cadence per instance
     for (int r = 0; r < reps; ++r) {
@@ -308,6 +322,7 @@ mf_status mf_batch_autotune(mf_context *ctx, const mf_csr *inst, int32_t k, int3
       ms += res.solve_ms / reps;
       ++n;
     }
+    lds = mf::batch_in_lds(resident);
     return MF_OK;
   };
   const mf_status st = descend(o, o.tile_lanes == 0, true, run, best, best_ms);

@@ -72,6 +72,10 @@ mf_status batch_upload(mf_context *ctx, const mf_csr *packed, const int32_t *src
 mf_status batch_solve_resident(mf_context *ctx, BatchResident *r, const mf_options &o,
                                int64_t *values, mf_result *res);
 void batch_release(BatchResident *r);
+// Whether the last solve ran inside one workgroup (every instance of the batch in one of its own), where
+// the options of the grid-wide kernels have no effect.
+bool batch_in_lds(const BatchResident *r);
+bool graph_in_lds(const mf_graph *g);
 
 // ---- serving arena: a device arena of vertex and slot ranges, and a persistent serving kernel
 // that solves the instances the host publishes into a queue while it runs (k_serve_wg) ----

@@ -2758,6 +2758,7 @@ struct DevGraph {
   std::vector<int32_t> h_off, h_dst, h_cap, h_fslot, h_src, h_snk;
   std::vector<int32_t> degree;  // residual slots of every vertex (out + in arcs)
   bool solved = false;
+  bool in_lds = false;  // the last solve ran in the LDS kernels alone (graph_in_lds)
   bool fresh = false;  // residuals still equal the capacities (built, not solved since)
   unsigned char *dirty = nullptr;  // BCSR/BCSR2 lines of slot pairs pushes changed (large graphs)
   int *bu_rem = nullptr;  // two lists of unreached vertices (2 x nonzero) + their class table
@@ -3181,6 +3182,7 @@ static mf_status run_one_workgroup(mf_context *ctx, DevGraph &G, const L &lay, c
     return MF_OK;
   }
   *taken = true;
+  G.in_lds = true;
   G.fresh = false;
   const mf_status status = r.status == 0 ? MF_OK
                            : r.status == 1 ? MF_ERR_ITERATION_LIMIT : MF_ERR_INTERNAL;
@@ -3414,6 +3416,7 @@ static mf_status run_solve(mf_context *ctx, DevGraph &G, const L &lay, mf_algo a
                                             G.m);
   }
   G.fresh = false;
+  G.in_lds = false;
   HIP_TRY(hipMemsetAsync(G.stats, 0, sizeof(unsigned long long) * kStatSlot * kStatSpread, st));
   HIP_TRY(hipMemsetAsync(G.ctl, 0, sizeof(int) * CTL_SIZE, st));
   const int pgrid = (int)std::min<int64_t>(16 * ctx->num_cu,
@@ -3977,6 +3980,7 @@ static mf_status run_batch_wg(mf_context *ctx, DevGraph &G, const int32_t *vbase
     res->status = result;
   }
   G.solved = result == MF_OK;
+  G.in_lds = huge == 0;
   return result;
 }
 
@@ -4063,6 +4067,8 @@ mf_status batch_solve_resident(mf_context *ctx, BatchResident *r, const mf_optio
   }
   return st;
 }
+
+bool batch_in_lds(const BatchResident *r) { return r->G.in_lds; }
 
 void batch_release(BatchResident *r) {
   if (!r) return;
@@ -4538,6 +4544,8 @@ static mf_status upload_static(mf_context *ctx, const mf_csr *c, DevGraph &G) {
 struct mf_graph {
   mf::DevGraph g;
 };
+
+bool mf::graph_in_lds(const mf_graph *g) { return g->g.in_lds; }
 
 // From this many vertices mf_graph_read_cut compares on the device and copies a byte per vertex
 // (R-MAT 22: 2.2 -> 0.34 ms, 79,000 vertices 58 -> 41 us); below, a launch costs what the smaller
