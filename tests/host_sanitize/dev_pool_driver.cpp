@@ -85,8 +85,28 @@ static int fits() {
   return 0;
 }
 
+// A full list makes room for what is used now: the second round of the same sizes allocates nothing.
+static int a_full_list_makes_room() {
+  hip_capacity = size_t(1) << 40;
+  mf::DevPool pool;
+  pool.set_limit(64 << 20, 32 << 20);
+  void *p[6];
+  for (size_t bytes : {size_t(10) << 20, size_t(8) << 20}) {
+    for (int round = 0; round < 2; ++round) {
+      const size_t before = hip_allocations;
+      for (void *&x : p) CHECK(pool.alloc(&x, bytes) == hipSuccess);
+      CHECK(round == 0 || hip_allocations == before);
+      for (void *x : p) pool.release(x);
+      CHECK(hip_held <= 64 << 20);
+    }
+  }
+  pool.trim();
+  CHECK(hip_held == 0);
+  return 0;
+}
+
 int main() {
   for (unsigned seed = 0; seed < 8; ++seed)
     if (random_calls(size_t(1) << (18 + seed), size_t(1) << (16 + 2 * seed), seed)) return 1;
-  return allocation_beside_another() || fits();
+  return allocation_beside_another() || fits() || a_full_list_makes_room();
 }

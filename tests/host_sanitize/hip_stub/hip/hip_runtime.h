@@ -6,7 +6,7 @@
 
 enum hipError_t { hipSuccess = 0, hipErrorOutOfMemory = 2 };
 
-inline size_t hip_capacity = 0, hip_held = 0;
+inline size_t hip_capacity = 0, hip_held = 0, hip_allocations = 0;
 inline std::map<void *, size_t> hip_blocks;
 
 inline hipError_t hipMalloc(void **p, size_t bytes) {
@@ -14,6 +14,7 @@ inline hipError_t hipMalloc(void **p, size_t bytes) {
   *p = std::malloc(1);
   hip_blocks[*p] = bytes;
   hip_held += bytes;
+  ++hip_allocations;
   return hipSuccess;
 }
 inline hipError_t hipFree(void *p) {

@@ -5,8 +5,8 @@
 // one another's kernels and for the serving kernel.  Freed blocks of up to max_block bytes go to a
 // list by size instead and are used again, by arrays of up to an eighth less.  The memory beyond what
 // the arrays in use need -- blocks on the list, and the ends of larger blocks in use -- stays within
-// the limit; what does not is given back at once, the rest with the context, or when an allocation
-// fails: then every context of the process gives its list back first.  A context
+// the limit: the blocks longest on the list are given back for a new one, the rest with the context,
+// or when an allocation fails: then every context of the process gives its list back first.  A context
 // belongs to one host thread at a time, and its calls end with their stream idle: a block on the
 // list has no work in flight.  The lock is for handles that another thread destroys (a garbage
 // collector's), as hipFree allowed, also while a call on other handles of the context runs.
@@ -14,6 +14,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstddef>
 #include <map>
 #include <mutex>
@@ -40,12 +41,12 @@ class DevPool {
     const size_t need = (bytes + 511) / 512 * 512;
     {
       std::lock_guard<std::mutex> lock(mutex_);
-      const auto it = kept_.lower_bound(need);
-      if (it != kept_.end() && it->first <= need + need / 8) {
-        *p = it->second;
-        used_[*p] = Block{it->first, need};
+      for (auto it = kept_.lower_bound(need); it != kept_.end() && it->first <= need + need / 8; ++it) {
+        if (it->second.empty()) continue;
+        *p = it->second.back();
+        it->second.pop_back();
+        blocks_[*p].need = need;
         spare_ -= need;
-        kept_.erase(it);
         return hipSuccess;
       }
     }
@@ -57,43 +58,40 @@ class DevPool {
     }
     if (e == hipSuccess) {
       std::lock_guard<std::mutex> lock(mutex_);
-      used_[*p] = Block{need, need};
+      blocks_[*p] = Block{need, need, 0};
     }
     return e;
   }
 
   // p: from alloc, with no device work on it in flight.
   void release(void *p) {
+    std::vector<void *> out;
     {
       std::lock_guard<std::mutex> lock(mutex_);
-      const auto it = used_.find(p);
-      if (it != used_.end()) {
-        const Block b = it->second;
-        used_.erase(it);
-        if (b.size <= max_block_ && spare_ + b.need <= limit_) {
-          kept_.emplace(b.size, p);
-          spare_ += b.need;
-          return;
-        }
-        spare_ -= b.size - b.need;
+      const auto it = blocks_.find(p);
+      if (it == blocks_.end()) {
+        out.push_back(p);
+      } else {
+        Block &b = it->second;
+        spare_ += b.need;
+        b.released = ++releases_;
+        kept_[b.size].push_back(p);
+        if (b.size > max_block_ || b.need > limit_) give_back(kept_.find(b.size), p, out);
+        shrink(out);
       }
     }
-    (void)hipFree(p);
+    for (void *x : out) (void)hipFree(x);
   }
 
-  // The largest blocks go first.
   void set_limit(size_t limit, size_t max_block) {
     std::vector<void *> out;
     {
       std::lock_guard<std::mutex> lock(mutex_);
       limit_ = limit;
       max_block_ = max_block;
-      while (!kept_.empty() && (spare_ > limit_ || std::prev(kept_.end())->first > max_block_)) {
-        const auto it = std::prev(kept_.end());
-        out.push_back(it->second);
-        spare_ -= it->first;
-        kept_.erase(it);
-      }
+      for (auto it = kept_.upper_bound(max_block_); it != kept_.end(); ++it)
+        while (!it->second.empty()) give_back(it, it->second.back(), out);
+      shrink(out);
     }
     for (void *p : out) (void)hipFree(p);
   }
@@ -102,10 +100,8 @@ class DevPool {
     std::vector<void *> out;
     {
       std::lock_guard<std::mutex> lock(mutex_);
-      for (const auto &b : kept_) {
-        out.push_back(b.second);
-        spare_ -= b.first;
-      }
+      for (auto it = kept_.begin(); it != kept_.end(); ++it)
+        while (!it->second.empty()) give_back(it, it->second.back(), out);
       kept_.clear();
     }
     for (void *p : out) (void)hipFree(p);
@@ -114,7 +110,37 @@ class DevPool {
  private:
   struct Block {
     size_t size, need;
+    unsigned long long released;  // when it went to the list
   };
+  using Kept = std::map<size_t, std::vector<void *>>;
+
+  // Takes p off the list (lock held).
+  void give_back(Kept::iterator it, void *p, std::vector<void *> &out) {
+    std::vector<void *> &v = it->second;
+    v.erase(std::find(v.begin(), v.end(), p));
+    spare_ -= it->first;
+    blocks_.erase(p);
+    out.push_back(p);
+  }
+
+  // Gives the oldest blocks back until the limit holds, or none is left (lock held).
+  void shrink(std::vector<void *> &out) {
+    while (spare_ > limit_) {
+      auto oldest = kept_.end();
+      void *p = nullptr;
+      unsigned long long when = ~0ull;
+      for (auto it = kept_.begin(); it != kept_.end(); ++it)
+        for (void *x : it->second)
+          if (blocks_[x].released < when) {
+            when = blocks_[x].released;
+            oldest = it;
+            p = x;
+          }
+      if (!p) return;
+      give_back(oldest, p, out);
+    }
+  }
+
   struct Registry {
     std::mutex mutex;
     std::set<DevPool *> pools;
@@ -129,9 +155,10 @@ class DevPool {
   }
 
   std::mutex mutex_;
-  std::multimap<size_t, void *> kept_;        // by size
-  std::unordered_map<void *, Block> used_;
-  size_t spare_ = 0;  // bytes held and not needed
+  Kept kept_;                                // by size
+  std::unordered_map<void *, Block> blocks_;  // every block, in use or kept
+  size_t spare_ = 0;                         // bytes held and not needed
+  unsigned long long releases_ = 0;
   size_t limit_ = size_t(256) << 20;
   size_t max_block_ = size_t(32) << 20;
 };
