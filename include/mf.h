@@ -100,7 +100,7 @@ typedef struct mf_options {
   int32_t bfs_block_frontier; /* frontier size up to which the one-workgroup BFS runs; 0 = default
                                  (its variant for graphs of low degree: eight times this) */
   float relabel_time_ratio;   /* adaptive cadence: after a global relabel taking T ms, cycles run
-                                 for about ratio * T ms; 0 = default (2) */
+                                 for about ratio * T ms; 0 = default (2.2, 2 inside one workgroup) */
   int32_t batch_algo;         /* mf_batch_solve, batch_mode 1 and instances of more than 2^19 vertices:
                                  0 = TC (default), 1 = VC */
   int32_t batch_mode;         /* mf_batch_solve: 0 = one workgroup per instance (default),

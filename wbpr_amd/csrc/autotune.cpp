@@ -62,8 +62,9 @@ const int32_t kForwardHops[] = {-1, 2, 8, 32};
 const int32_t kFrontiers[] = {256, 1024, 4096, 16384};
 const double kCadenceFactors[] = {1.0, 1.5, 2.0};
 
-float effective_ratio(const mf_options &o) {
-  return o.relabel_time_ratio > 0 ? o.relabel_time_ratio : 2.0f;
+float effective_ratio(const mf_options &o, bool lds) {
+  if (o.relabel_time_ratio > 0) return o.relabel_time_ratio;
+  return lds ? mf::kLdsRelabelRatio : mf::kGridRelabelRatio;
 }
 
 int32_t effective_frontier(const mf_options &o) {
@@ -115,7 +116,7 @@ mf_status sweep(const mf_options &cur, const bool &lds, bool tune_lanes, bool tu
     if ((st = consider(t)) != MF_OK) return st;
   }
   if (cur.cycles_per_relabel == 0) {  // the time ratio only steers the adaptive cadence
-    const float r0 = effective_ratio(cur);
+    const float r0 = cur.relabel_time_ratio;
     for (float r : kRatios) {
       if (r == r0) continue;
       mf_options t = cur;
@@ -161,7 +162,6 @@ template <class Run>
 mf_status descend(mf_options cur, bool tune_lanes, bool tune_batch_algo, Run run,
                   mf_options *best, double *best_ms) {
   // the result names every tuned value explicitly (0 would mean "library default")
-  cur.relabel_time_ratio = effective_ratio(cur);
   cur.bfs_block_frontier = effective_frontier(cur);
   if (cur.forward_hops == 0) cur.forward_hops = 2;
   if (tune_lanes)
@@ -185,6 +185,7 @@ mf_status descend(mf_options cur, bool tune_lanes, bool tune_batch_algo, Run run
   double cadence_base = 0;
   mf_status st = time_cur(2 * kRepeats, &cadence_base);
   if (st != MF_OK) return st;
+  cur.relabel_time_ratio = effective_ratio(cur, lds);
   const mf_options start = cur;
   bool changed = false;
   auto consider = [&](const mf_options &t) -> mf_status {

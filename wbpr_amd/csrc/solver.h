@@ -40,6 +40,9 @@ mf_status batch_solve_packed(mf_context *ctx, const mf_csr *packed, const int32_
                              mf_layout layout, const mf_options &o, int64_t *values,
                              mf_result *res);
 
+// mf_options.relabel_time_ratio 0, for solves inside one workgroup and for the others.
+constexpr float kLdsRelabelRatio = 2.0f, kGridRelabelRatio = 2.2f;
+
 // Whether a solve that returns only a value takes the reversed network: clearly less capacity into
 // the sink than out of the source (pack_instances).  Less than an eighth apart nothing is gained.
 inline bool solves_reversed(int64_t from_s, int64_t into_t) { return into_t < from_s - from_s / 8; }

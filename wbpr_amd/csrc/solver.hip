@@ -2559,7 +2559,12 @@ static double now_ms() {
 // stay balanced whether relabels are cheap (small graphs) or dominated by long BFS chains.
 // Excess that can no longer reach a sink only stops moving at the next global relabel, which is
 // why a fixed large cycle count is wasteful on graphs that strand excess (bipartite, RLG).
-constexpr float kDefaultRelabelRatio = 2.0f;
+//
+// 2 inside one workgroup, where 0.5 to 8 were swept.  2.2 on the grid: its relabels became 5 to 10%
+// shorter when a read-back between their levels went, and with 2 the cycles' time did too, so that
+// graphs whose flow just arrived in two rounds took a third (R-MAT 13, edge factor 16: 0.77 -> 1.46 ms).
+// 58 R-MAT graphs of scale 12 to 19 against the time before: 0.73 to 0.78 of the speed at worst and 1.04 on
+// average with 2, 0.89 and 1.10 with 2.2, 0.84 and 1.13 with 2.3; 40 matchings 1.09 and 1.08 on average.
 constexpr int kMaxAdaptiveCycles = 1 << 14;  // cap of cycles per round in adaptive mode
 constexpr int kDefaultBfsFrontier = 4096;    // one-workgroup BFS up to this frontier size
 constexpr int kWgBfsSlots = 32768;           // ... and up to about this many frontier slots
@@ -3158,7 +3163,7 @@ static mf_status run_one_workgroup(mf_context *ctx, DevGraph &G, const L &lay, c
   a.n = G.n;
   a.s = G.h_src[0];
   a.t = G.h_snk[0];
-  a.ratio = o.relabel_time_ratio > 0 ? o.relabel_time_ratio : kDefaultRelabelRatio;
+  a.ratio = o.relabel_time_ratio > 0 ? o.relabel_time_ratio : kLdsRelabelRatio;
   if (o.cycles_per_relabel > 0) a.ratio = 1e30f;  // fixed cadence: only the count ends a round
   a.max_cycles = o.cycles_per_relabel > 0 ? o.cycles_per_relabel : kMaxAdaptiveCycles;
   a.max_rounds = o.max_rounds > 0 ? o.max_rounds : (int64_t)100000000;
@@ -3348,7 +3353,7 @@ static mf_status run_solve(mf_context *ctx, DevGraph &G, const L &lay, mf_algo a
   bool use_coop = ctx->cooperative && o.bfs_cooperative == 1;
   const bool adaptive = o.cycles_per_relabel == 0;
   const int K = adaptive ? kMaxAdaptiveCycles : o.cycles_per_relabel;
-  const double ratio = o.relabel_time_ratio > 0 ? o.relabel_time_ratio : kDefaultRelabelRatio;
+  const double ratio = o.relabel_time_ratio > 0 ? o.relabel_time_ratio : kGridRelabelRatio;
   double last_relabel_ms = 0;
   double cyc_est_ms = 0;  // wall time per cycle launch in the last chunk
   // captured cycle chunks, one per length (multiples of kGraphPeriod), cached on the graph for
@@ -3898,7 +3903,7 @@ static mf_status run_batch_wg(mf_context *ctx, DevGraph &G, const int32_t *vbase
     b.blanes[c] = vc.lanes[c];
   }
   b.use_vcls = cc.nclass > 1;
-  b.ratio = o.relabel_time_ratio > 0 ? o.relabel_time_ratio : kDefaultRelabelRatio;
+  b.ratio = o.relabel_time_ratio > 0 ? o.relabel_time_ratio : kLdsRelabelRatio;
   b.max_rounds = o.max_rounds > 0 ? (int)std::min<int64_t>(o.max_rounds, INT32_MAX) : 1000000;
   b.max_cycles = o.cycles_per_relabel > 0 ? o.cycles_per_relabel : kMaxAdaptiveCycles;
   b.fwd_hops = o.forward_hops < 0 ? 0 : (o.forward_hops > 0 ? o.forward_hops : kDefaultForwardHops);
@@ -4403,7 +4408,7 @@ mf_status serve_launch(ServeArena *a) {
   sa.qcap = a->qcap;
   sa.idle_ticks = kServeIdleTicks;
   sa.lds_bytes = kServeLds;
-  sa.wg_ratio = kDefaultRelabelRatio;
+  sa.wg_ratio = kLdsRelabelRatio;
   HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(k_serve_wg<LayoutBCSR>),
                               hipFuncAttributeMaxDynamicSharedMemorySize, kServeLds));
   k_serve_wg<LayoutBCSR><<<a->groups, kBlock, kServeLds, a->kernel_stream>>>(
