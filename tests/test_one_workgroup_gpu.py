@@ -142,7 +142,8 @@ def test_grid_goes_on_from_an_abandoned_search(mf, orc, ctx, width, length, coop
 
 
 @pytest.mark.parametrize("left,right,both_lines", [
-    (9200, 9150, True), (9250, 9201, False),      # the sink takes less: frontiers up to 9,200 stay
+    (9600, 9400, True), (9600, 9401, False),      # the sink takes less: frontiers up to 9,400 stay
+    (9600, 9550, True),                          # (hardly less)
     (11400, 11800, True), (11400, 11801, False),  # more: up to 11,800
 ])
 def test_wide_frontiers_by_layout(mf, orc, ctx, left, right, both_lines):

@@ -42,6 +42,7 @@ __device__ __forceinline__ void st_rel(int *p, int v) {
 // so the next solve restores only those lines to the capacities.  Null: not tracked.
 struct LayoutBCSR {
   static constexpr int kSeg = 1;
+  static constexpr bool kOneLine = true;  // a slot and its residual are one record
   const int *off;
   int2 *dc;
   const int *rev;
@@ -96,6 +97,7 @@ struct LayoutBCSR {
 // BCSR2 (maxflow-bcsr2 layout): dst array plus interleaved {residual, reverse slot} pairs.
 struct LayoutBCSR2 {
   static constexpr int kSeg = 1;
+  static constexpr bool kOneLine = false;
   const int *off;
   const int *dst;
   int2 *cr;
@@ -146,6 +148,7 @@ struct LayoutBCSR2 {
 // direction, m + k for reverse position k.
 struct LayoutRCSR {
   static constexpr int kSeg = 2;
+  static constexpr bool kOneLine = false;
   const int *off;
   int2 *fdc;
   int *bcf;

@@ -2470,7 +2470,7 @@ __global__ __launch_bounds__(kBlock) void k_serve_wg(L g, ServeArgs a) {
       w.st = WgStats{0, 0, 0, 0, 0, 0};
       w.carve(lds, a.lds_bytes, nullptr, nullptr);
       const WgOutcome o = w.solve(a.wg_ratio, a.b.max_cycles, a.b.max_rounds,
-                                  WgWide{s_entry[5], 0, INT_MAX, INT_MAX});
+                                  WgWide{s_entry[5], 0, 0, 0});
       value = o.value;
       status = o.status;
       st = Stats{w.st.active, w.st.slots, w.st.pushes, w.st.relabels};
@@ -3111,14 +3111,14 @@ static void restore_residuals(mf_context *ctx, DevGraph &G) {
 // grid; with the excesses in global memory none (16,000 + 16,000: 3.9 and 3.2 ms, 20,000 + 20,500: 2.3
 // and 2.8 ms, Genrmf 48 x 48 x 20: 32 and 40 ms).  BCSR reads a slot from one line; RCSR and BCSR2, which
 // read two, keep one CU's memory path busy sooner: their wide frontiers stay up to kWgWideMost vertices,
-// up to kWgWideShort where the sink takes less than the source gives and the rest moves about until
-// a relabel finds it cut off.  (RCSR matchings, grid and here: 9,000 x 8,640 1.89 and 1.73 ms, 10,000
+// up to kWgWideShort where the sink takes a 64th less than the source gives and the rest moves about
+// until a relabel finds it cut off.  (RCSR matchings, grid and here: 9,000 x 8,640 1.89 and 1.73 ms, 10,000
 // x 9,600 1.84 and 2.02, 12,000 x 11,520 1.91 and 2.57; 11,000 x 11,440 1.69 and 1.52, 12,000 x 12,480
 // 1.75 and 2.00.  BCSR 12,000 x 11,520 1.85 and 1.48.)
 constexpr int64_t kWgNarrowSlots = 1 << 16;
 constexpr int64_t kWgMaxSlots = 1 << 21;
 constexpr int kWgWideBoth = 2800, kWgWideHeights = 2048;
-constexpr int kWgWideLevels = 2, kWgWideMost = 11800, kWgWideShort = 9200;
+constexpr int kWgWideLevels = 2, kWgWideMost = 11800, kWgWideShort = 9400;
 
 // At most an eighth of the slots belong to vertices of more than 32.
 static bool low_degree(const DevGraph &G) { return G.heavy_slots * 8 <= 2 * G.m; }
@@ -3170,9 +3170,8 @@ static mf_status run_one_workgroup(mf_context *ctx, DevGraph &G, const L &lay, c
   const bool both = kind == kWgBoth;
   a.wide = kWgNeverWide;
   if (slots > kWgNarrowSlots)
-    a.wide = !both                         ? WgWide{kWgWideHeights, 0, INT_MAX, INT_MAX}
-             : G.layout == MF_LAYOUT_BCSR ? WgWide{kWgWideBoth, kWgWideLevels, INT_MAX, INT_MAX}
-                                           : WgWide{kWgWideBoth, kWgWideLevels, kWgWideMost, kWgWideShort};
+    a.wide = both ? WgWide{kWgWideBoth, kWgWideLevels, kWgWideMost, kWgWideShort}
+                  : WgWide{kWgWideHeights, 0, INT_MAX, INT_MAX};
   a.values = G.values;
   static_assert(sizeof(WgReport) <= sizeof(int) * CTL_SIZE, "the report fits the control words");
   a.report = reinterpret_cast<WgReport *>(G.ctl);  // the grid-wide kernels' words, free here

@@ -11,8 +11,8 @@ namespace mfk {
 enum WgKind { kWgBoth = 0, kWgHeights = 1, kWgGlobal = 2 };  // see wg_solve.h
 
 // When the first global relabel gives a solve up: once more than `levels` frontiers held more than
-// `from` vertices (0: never), or one more than `most` -- more than `most_short` where the sink takes
-// less than the source gives.
+// `from` vertices (0: never); on layouts that read two lines for a slot also at one of more than
+// `most` -- of more than `most_short` where the sink takes a 64th less than the source gives.
 struct WgWide {
   int from, levels, most, most_short;
 };

@@ -18,6 +18,7 @@
 // excess instead of by the list.
 #pragma once
 
+#include <cstddef>
 #include <type_traits>
 
 #include "kernels.h"
@@ -56,12 +57,11 @@ __host__ __device__ constexpr int wg_kind(long long n, long long room) {
   return -1;
 }
 
-struct WgShared {
+struct alignas(8) WgShared {
   int cnt[3];   // items of the list a cycle or level reads (q % 3), fills ((q + 1) % 3), clears
   int nhub[3];  // hubs waiting, same rotation
   int chunk;    // items of the chunk list while an overflowed worklist is walked
   int flag;     // a source was reached
-  long long surplus;
   int stop[2];
   int hub[2][kWgHubCap];
 };
@@ -482,35 +482,36 @@ struct WgSolver {
     expand<B>(u, r, lane, T, level, check, out, ocnt);
   }
 
-  // Capacity out of the source less capacity into the sink.
-  __device__ __forceinline__ long long surplus() {
+  // Whether less than 63 / 64 of the capacity out of the source goes into the sink.
+  __device__ __forceinline__ bool short_sink() {
     const int tid = (int)threadIdx.x;
-    if (tid == 0) S.surplus = 0;
+    auto *surplus = reinterpret_cast<unsigned long long *>(S.hub[0]);  // (no hubs yet)
+    static_assert(offsetof(WgShared, hub) % 8 == 0, "a 64-bit word");
+    if (tid == 0) *surplus = 0;
     __syncthreads();
     long long sum = 0;
     Range r = range(s);
     for (int i = tid; i < r.d; i += BS) {
       int w, res, key;
       g.scan(r.seg(i), r.at(i), w, res, key);
-      if (w - vb != s) sum += res;
+      if (w - vb != s) sum += 63LL * res;
     }
     r = range(t);
     for (int i = tid; i < r.d; i += BS) {
       int w, idx;
       g.bfs_slot(r.seg(i), r.at(i), w, idx);
-      if (w - vb != t) sum -= g.bfs_rin(r.seg(i), idx);
+      if (w - vb != t) sum -= 64LL * g.bfs_rin(r.seg(i), idx);
     }
     sum = tile_sum<64>(sum);
-    if (__lane_id() == 0)
-      atomicAdd(reinterpret_cast<unsigned long long *>(&S.surplus), (unsigned long long)sum);
+    if (__lane_id() == 0) atomicAdd(surplus, (unsigned long long)sum);
     __syncthreads();
-    return S.surplus;
+    return (long long)*surplus > 0;
   }
 
   // Heights from a BFS over reverse residual arcs: distances to the sink, n where it cannot be
-  // reached.  Returns the levels; wide.from > 0 gives up (WgWide), before anything outside LDS has been
+  // reached.  Returns the levels; from > 0 gives up (see WgWide), before anything outside LDS has been
   // written: -1 - level, the heights up to that level set.
-  __device__ __forceinline__ int relabel(const WgWide &wide, bool check) {
+  __device__ __forceinline__ int relabel(int from, int levels, int most, bool check) {
     const int tid = (int)threadIdx.x;
     for (int v = tid; v < n; v += BS) h[v] = (HT)(v == s ? n + 1 : (v == t ? 0 : n));
     for (int w = tid; w < wg_bits_words(n); w += BS) {
@@ -528,12 +529,15 @@ struct WgSolver {
       list(0)[0] = (HT)t;
     }
     __syncthreads();
-    int level = 0, left = wide.levels, most = wide.most;
-    if (wide.from > 0 && wide.most_short < wide.most && surplus() > 0) most = wide.most_short;
+    int level = 0;
     for (;; ++level) {
       const int cnt = S.cnt[level % 3];
       if (cnt == 0) break;
-      if (wide.from > 0 && cnt > wide.from && (cnt > most || left-- == 0)) return -1 - level;
+      if (from > 0 && cnt > from) {
+        if constexpr (!L::kOneLine)
+          if (cnt > most) return -1 - level;
+        if (levels-- == 0) return -1 - level;
+      }
       if (tid == 0) {
         S.cnt[(level + 2) % 3] = 0;
         // (filled in the level that uses it, and read after that level's barrier: the next level's
@@ -574,6 +578,9 @@ struct WgSolver {
   __device__ __forceinline__ WgOutcome solve(float ratio, int max_cycles, long long max_rounds,
                                              const WgWide &wide) {
     const int tid = (int)threadIdx.x;
+    int most = 0;
+    if constexpr (!L::kOneLine)
+      if (wide.from > 0) most = short_sink() ? wide.most_short : wide.most;
     WgOutcome o{0, 0, 0, 0, 0, 0, 0, 0};
     if constexpr (KIND == kWgBoth) {
       for (int v = tid; v < n; v += BS) e[v] = 0;
@@ -589,7 +596,7 @@ struct WgSolver {
         break;
       }
       const long long t0 = (long long)wall_clock64();
-      const int levels = relabel(round == 0 ? wide : kWgNeverWide, round > 0);
+      const int levels = relabel(round == 0 ? wide.from : 0, wide.levels, most, round > 0);
       if (levels < 0) {
         o.status = 3;
         o.levels = -1 - levels;

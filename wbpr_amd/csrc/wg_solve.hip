@@ -42,14 +42,16 @@ __device__ __forceinline__ void write_report(WgReport *rep, const WgOutcome &o, 
 
 // A single graph.  Its heights and excesses go to global memory at the end, where the read-back
 // entry points, or a global relabel that goes on from an abandoned one, expect them.
-template <class L, int KIND>
+// WIDE: the first global relabel may give up.
+template <class L, int KIND, bool WIDE>
 __global__ __launch_bounds__(kWgThreads) void k_wg_solve(L g, WgSingle a) {
   extern __shared__ __align__(16) char lds[];
   __shared__ WgShared S;
   WgSolver<L, KIND, kWgThreads> w{g, S, 0, a.n, a.s, a.t};
   w.st = WgStats{0, 0, 0, 0, 0, 0};
   w.carve(lds, a.lds_bytes, a.h, a.e);
-  const WgOutcome o = w.solve(a.ratio, a.max_cycles, a.max_rounds, a.wide);
+  const WgOutcome o = w.solve(a.ratio, a.max_cycles, a.max_rounds,
+                              WIDE ? a.wide : kWgNeverWide);
   for (int v = (int)threadIdx.x; v < a.n; v += kWgThreads) {
     a.h[v] = w.h[v];
     if constexpr (KIND == kWgBoth) a.e[v] = w.e[v];
@@ -65,13 +67,13 @@ int wg_single_kind(int32_t n, int lds_limit) {
 
 // (The attribute is the kernel's, not the launch's: every thread sets the same value, not its own
 // launch's size, which another thread's smaller graph could lower before the launch.)
-template <class L, int KIND>
+template <class L, int KIND, bool WIDE>
 static hipError_t launch_single(hipStream_t st, const L &g, const WgSingle &a, int lds_limit) {
   const hipError_t e =
-      hipFuncSetAttribute(reinterpret_cast<const void *>(k_wg_solve<L, KIND>),
+      hipFuncSetAttribute(reinterpret_cast<const void *>(k_wg_solve<L, KIND, WIDE>),
                           hipFuncAttributeMaxDynamicSharedMemorySize, lds_limit - kWgStaticLds);
   if (e != hipSuccess) return e;
-  k_wg_solve<L, KIND><<<1, kWgThreads, a.lds_bytes, st>>>(g, a);
+  k_wg_solve<L, KIND, WIDE><<<1, kWgThreads, a.lds_bytes, st>>>(g, a);
   return hipGetLastError();
 }
 
@@ -79,8 +81,11 @@ template <class L>
 hipError_t wg_single_launch(hipStream_t st, const L &g, WgSingle a, int kind, int lds_limit) {
   const long long all = wg_state_bytes(kind, a.n) + 2LL * wg_item_bytes(kind) * a.n;
   a.lds_bytes = (int)std::min<long long>((all + 15) / 16 * 16, lds_limit - kWgStaticLds);
-  return kind == kWgBoth ? launch_single<L, kWgBoth>(st, g, a, lds_limit)
-                         : launch_single<L, kWgHeights>(st, g, a, lds_limit);
+  if (a.wide.from > 0)
+    return kind == kWgBoth ? launch_single<L, kWgBoth, true>(st, g, a, lds_limit)
+                           : launch_single<L, kWgHeights, true>(st, g, a, lds_limit);
+  return kind == kWgBoth ? launch_single<L, kWgBoth, false>(st, g, a, lds_limit)
+                         : launch_single<L, kWgHeights, false>(st, g, a, lds_limit);
 }
 template hipError_t wg_single_launch(hipStream_t, const LayoutBCSR &, WgSingle, int, int);
 template hipError_t wg_single_launch(hipStream_t, const LayoutBCSR2 &, WgSingle, int, int);
