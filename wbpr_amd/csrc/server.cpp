@@ -7,9 +7,9 @@
 //     serving kernel (k_serve_wg) that keeps running while requests arrive.  A workgroup of the
 //     running kernel takes it as soon as one is free, so requests that arrive while others are on
 //     the GPU join the running batch; their ranges are freed and reused as they finish.
-//   - alone (larger requests): one workgroup would take tens of milliseconds on them, so each
-//     runs on the whole grid (the single-instance solver) from a worker thread with its own
-//     context and stream, overlapping on the device with the serving kernel and other large
+//   - alone (larger requests): each is a single solve (inside one workgroup with a CU's whole LDS, or on
+//     the grid) from a worker thread with its own context and stream, overlapping on the device
+//     with the serving kernel, which leaves CUs and hardware queues for them, and with other large
 //     requests.  Its device memory is charged to the budget, and kept for the next request as far as
 //     the requests in flight leave room.
 // The budget (hbm_budget_bytes) is split: half for the arena, half for the large requests in
@@ -35,7 +35,7 @@ using namespace mf;
 
 namespace {
 
-// Requests above either size run alone on the whole grid.
+// Requests above either size run alone.
 constexpr int32_t kSoloVertices = kServeVertices;
 constexpr int64_t kSoloArcs = 262144;
 constexpr int32_t kQueueCap = 4096;    // entries of the serving kernel's queue ring
@@ -85,7 +85,7 @@ struct Request {
   }
 };
 
-// A large request solved alone on the whole grid by a worker thread.
+// A large request solved alone by a worker thread.
 struct Launch {
   std::shared_ptr<Request> req;
   int ctx_slot = -1;
@@ -228,7 +228,7 @@ static void run_alone(mf_server *srv, Launch *L) {
   mf_result res{};
   int64_t value = 0;
   const int32_t src = r.s, snk = r.t, vbase[2] = {0, r.n};
-  o.batch_mode = 1;  // the grid-wide single-instance solver
+  o.batch_mode = 1;  // as a single graph
   const mf_status stt = batch_solve_packed(srv->ctxs[(size_t)L->ctx_slot], &c, &src, &snk, vbase,
                                            1, MF_ALGO_VC, MF_LAYOUT_BCSR, o, &value, &res);
   std::lock_guard<std::mutex> lk(srv->mu);
